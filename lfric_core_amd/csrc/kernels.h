@@ -37,6 +37,14 @@ int launch_op_convert(const lfric_op *src, lfric_op *dst);
 
 // operator kernels
 int launch_lma_apply(const lfric_op *op, const void *x, void *y, const int *d_skip);
+// the colour-ordered apply of an order-1 W0 operator (27 x 27 elements, W0 column roles), rows
+// split over threads; nrhs 1, 2, 4 or 8 (order1_apply.hip)
+int launch_colour_rows27(const lfric_op *op, const void *x, void *y, int nrhs, const int *skip);
+// whether it is the faster form: one right-hand side always; several where a level's x does not
+// fit the registers, or colours of at most 32768 units (the split then fills the GPU; beyond, one
+// thread per unit reads x once for all rows: C24x70, 2 FP64 right-hand sides 326 us against 347, and
+// C24x30, 26784 units, 206 against 179)
+bool colour_rows27_faster(const lfric_op *op, int nrhs);
 int launch_lma_apply_gather(const lfric_op *op, const void *x, void *y);
 // gather apply that also leaves one x.y partial sum per block in `partials` (square
 // operators); stops at once when *skip is set

@@ -2365,10 +2365,7 @@ static void launch_colour(RoleKind rk, int grid, const lfric_op *op, size_t S, c
         LAUNCH((k_lma_colour<T, A_, B_, RolesW0K0>), grid, Ad, S, to.d_ebase, x, y, to.d_map, from.d_map, first, pos0, npos, nl,
                RolesW0K0{}, d_skip, op->xwin);
       break;
-    case RoleKind::W0K1:
-      if constexpr (A_ == 27)
-        LAUNCH((k_lma_colour<T, A_, B_, RolesW0K1>), grid, Ad, S, to.d_ebase, x, y, to.d_map, from.d_map, first, pos0, npos, nl,
-               RolesW0K1{}, d_skip, op->xwin);
+    case RoleKind::W0K1:  // launch_colour_rows27
       break;
     case RoleKind::W2K0:
       if constexpr (A_ == 6)
@@ -2389,6 +2386,7 @@ template <typename T>
 static int apply_colours_t(const lfric_op *op, const T *x, T *y, const int *d_skip) {
   const FunctionSpace &to = *op->to, &from = *op->from;
   RoleKind rk = role_kind(to);
+  if (rk == RoleKind::W0K1 && from.ndf == 27) return launch_colour_rows27(op, x, y, 1, d_skip);
   const size_t S = op->gs;
   const int nl = to.nlayers;
   for (int c = 0; c < to.ncolours; ++c) {
@@ -2658,7 +2656,10 @@ static int launch_mrhs_n(int variant, RoleKind rk, const lfric_op *op, const T *
   if (variant == LFRIC_MRHS_COLOUR) {
     switch (rk) {
       case RoleKind::W0K0: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K0{}); break;
-      case RoleKind::W0K1: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K1{}); break;
+      case RoleKind::W0K1:
+        if (N1 == 27 && N2 == 27 && colour_rows27_faster(op, NR)) return launch_colour_rows27(op, x, y, NR, nullptr);
+        launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K1{});
+        break;
       case RoleKind::W2K0: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW2K0{}); break;
       case RoleKind::None: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesNone{}); break;
       default: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesRuntime{rr});
@@ -2749,8 +2750,12 @@ int launch_lma_apply_mrhs(const lfric_op *op, const void *x, void *y, int nrhs, 
     // copy; otherwise the colour-ordered form with register-staged x is the fastest from a few
     // hundred thousand cells up (C96x70 W0, 4 FP32 RHS: 0.310 ms vs gather 0.354); on small
     // meshes its one launch per colour leaves the GPU idle and the gather form wins
+    // (order 1: from 8000 cells, with its rows split over threads; C12x10, 4 FP32 RHS 30 us against 55,
+    // C6x20, 2 FP32 RHS 24 against 20; not 8 FP64 RHS, C24x30 702 us against 631)
     const long long nc3 = static_cast<long long>(op->to->ncells) * op->to->nlayers;
-    variant = (nrhs > 1 && nc3 >= 200000 && !op->rows && !sym27_ready(op)) ? LFRIC_MRHS_COLOUR : LFRIC_MRHS_GATHER;
+    const bool rows27 = role_kind(*op->to) == RoleKind::W0K1 && op->from->ndf == 27 &&
+                        !(op->precision == LFRIC_R64 && nrhs == 8);
+    variant = (nrhs > 1 && nc3 >= (rows27 ? 8000 : 200000) && !op->rows && !sym27_ready(op)) ? LFRIC_MRHS_COLOUR : LFRIC_MRHS_GATHER;
   }
   LF_CHECK(variant == LFRIC_MRHS_GATHER || variant == LFRIC_MRHS_COLOUR || variant == LFRIC_MRHS_MFMA, LFRIC_E_ARG,
            "unknown multi-RHS variant");
