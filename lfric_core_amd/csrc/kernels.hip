@@ -2653,26 +2653,38 @@ static void launch_colour_mrhs_r(const lfric_op *op, const T *x, T *y, R roles) 
 template <typename T, int N1, int N2, int NR>
 static int launch_mrhs_n(int variant, RoleKind rk, const lfric_op *op, const T *x, T *y) {
   const Roles rr = roles_of(*op->to);
-  if (variant == LFRIC_MRHS_COLOUR) {
-    switch (rk) {
-      case RoleKind::W0K0: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K0{}); break;
-      case RoleKind::W0K1:
-        if (N1 == 27 && N2 == 27 && colour_rows27_faster(op, NR)) return launch_colour_rows27(op, x, y, NR, nullptr);
-        launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K1{});
-        break;
-      case RoleKind::W2K0: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW2K0{}); break;
-      case RoleKind::None: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesNone{}); break;
-      default: launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesRuntime{rr});
+  const bool colour = variant == LFRIC_MRHS_COLOUR;
+  // each role table belongs to one element size
+  if constexpr (N1 == 8 && N2 == 8) {
+    if (rk == RoleKind::W0K0) {
+      if (!colour) return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW0K0{});
+      launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K0{});
+      return LFRIC_OK;
     }
+  }
+  if constexpr (N1 == 27 && N2 == 27) {
+    if (rk == RoleKind::W0K1) {
+      if (!colour) return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW0K1{});
+      if (colour_rows27_faster(op, NR)) return launch_colour_rows27(op, x, y, NR, nullptr);
+      launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW0K1{});
+      return LFRIC_OK;
+    }
+  }
+  if constexpr (N1 == 6 && N2 == 6) {
+    if (rk == RoleKind::W2K0) {
+      if (!colour) return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW2K0{});
+      launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesW2K0{});
+      return LFRIC_OK;
+    }
+  }
+  if (rk == RoleKind::None) {
+    if (!colour) return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesNone{});
+    launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesNone{});
     return LFRIC_OK;
   }
-  switch (rk) {
-    case RoleKind::W0K0: return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW0K0{});
-    case RoleKind::W0K1: return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW0K1{});
-    case RoleKind::W2K0: return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesW2K0{});
-    case RoleKind::None: return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesNone{});
-    default: return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesRuntime{rr});
-  }
+  if (!colour) return launch_gather_mrhs_r<T, N2, NR>(op, x, y, RolesRuntime{rr});
+  launch_colour_mrhs_r<T, N1, N2, NR>(op, x, y, RolesRuntime{rr});
+  return LFRIC_OK;
 }
 
 template <typename T, int NR>
