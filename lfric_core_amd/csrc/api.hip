@@ -56,6 +56,7 @@ FunctionSpace::~FunctionSpace() {
   dfree(d_gcol, gcol_bytes);
   dfree(d_goff, goff_bytes);
   dfree(d_gent, gent_bytes);
+  dfree(d_w0tab, w0tab_bytes);
 }
 
 // Scratch vectors of the solvers, kept between solves (grown on demand).  Slots: 0-2 CG's r, z,
@@ -740,6 +741,13 @@ int lfric_op_create(const lfric_fs *to, const lfric_fs *from, int precision, lfr
     return rc;
   }
   LF_HIP(hipMemsetAsync(op->d, 0, op->bytes, cur_stream()));
+  // the table of the lowest-order W0 apply, here so that the apply itself never allocates (it may be
+  // captured)
+  if (op->to == op->from)
+    if (int rc = build_w0_table(*op->to)) {
+      lfric_op_destroy(op);
+      return rc;
+    }
   *out = op;
   return LFRIC_OK;
 }

@@ -110,6 +110,11 @@ struct FunctionSpace {
   int *d_goff = nullptr;                   // [col+1] offsets into d_gent
   int *d_gent = nullptr;                   // pos * 32 + df
   size_t gcol_bytes = 0, goff_bytes = 0, gent_bytes = 0;
+  // lowest-order W0 spaces whose columns have at most 4 cells: the same lists, one entry per column
+  // (w0_apply.hip); null otherwise
+  void *d_w0tab = nullptr;
+  int w0tab_cols = 0;
+  size_t w0tab_bytes = 0;
   ~FunctionSpace();
 };
 

@@ -37,6 +37,14 @@ int launch_op_convert(const lfric_op *src, lfric_op *dst);
 
 // operator kernels
 int launch_lma_apply(const lfric_op *op, const void *x, void *y, const int *d_skip);
+// The gather lists of a lowest-order W0 space as one table entry per dof column (no table, with
+// LFRIC_OK, for other spaces and where a column has more than 4 cells), and the apply of a square
+// operator over it: the gather form's sums, or (colour) the colour-ordered form's, bit for bit;
+// w0_apply.hip.  The table is always the faster form, so there is no rule of sizes.
+int build_w0_table(FunctionSpace &f);
+int launch_w0_gather(const lfric_op *op, const void *x, void *y, bool colour, double *partials, const int *skip);
+// the space's gather lists, built on first use
+int prepare_gather(FunctionSpace &f);
 // the colour-ordered apply of an order-1 W0 operator (27 x 27 elements, W0 column roles), rows
 // split over threads; nrhs 1, 2, 4 or 8 (order1_apply.hip)
 int launch_colour_rows27(const lfric_op *op, const void *x, void *y, int nrhs, const int *skip);
@@ -67,6 +75,8 @@ int launch_build_sym(lfric_op *op, int levels_per_thread);
 void drop_sym(lfric_op *op);
 // the operator's symmetric-packed copy is the order-1 W0 kind (sym27_apply.h)
 bool sym27_ready(const lfric_op *op);
+// its apply of 2, 4 or 8 right-hand sides
+int launch_sym27_mrhs(const lfric_op *op, const void *x, void *y, int nrhs);
 int launch_assemble_mass_w0(lfric_op *op, const double *chi1, const double *chi2, const double *chi3, int nqp);
 // tridiagonal solve of every column of a square columnwise operator (columnwise_op_appinv)
 int launch_cma_appinv(const lfric_cma *A, const void *x, void *y);
