@@ -22,6 +22,7 @@ struct GmresState {
   double g[kMaxKrylov + 1];
   double u[kMaxKrylov];
   double cs[kMaxKrylov], sn[kMaxKrylov];  // the cycle's Givens rotations, formed column by column
+  double l[kMaxKrylov * kMaxKrylov];      // v_j . v_i at [i*kMaxKrylov + j], i < j (the basis' own products)
   double beta;
   double rnorm2;
   double beta0;  // beta of the first cycle
@@ -244,25 +245,14 @@ __global__ __launch_bounds__(kColThreads) void k_coltri_apply_tile(const typenam
 }
 
 // ---- GMRES -------------------------------------------------------------------------------
-// one fused modified Gram-Schmidt step j of Arnoldi column iv:
-//   j > 0      : w = w - h(j-1,iv) v_{j-1}
-//   j <= iv    : partial v_j . w          -> h(j,iv)
-//   j == iv+1  : partial w . w            -> h(iv+1,iv) = sqrt
+// block partials of a . b (a null: b . b)
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mgs_step(T *__restrict__ w, const T *__restrict__ vprev,
-                                                     const T *__restrict__ vj, long long n, const double *hprev,
-                                                     double *partials) {
-  const T a = hprev ? static_cast<T>(-*hprev) : T(0);
+__global__ __launch_bounds__(kBlock) void k_dot_partials(const T *__restrict__ a, const T *__restrict__ b, long long n,
+                                                         double *partials) {
   double v[1] = {0.0};
   for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<long long>(gridDim.x) * blockDim.x) {
-    T wi = w[i];
-    if (vprev) {
-      wi = wi + a * vprev[i];
-      w[i] = wi;
-    }
-    v[0] += vj ? to_d(vj[i]) * to_d(wi) : to_d(wi) * to_d(wi);
-  }
+       i += static_cast<long long>(gridDim.x) * blockDim.x)
+    v[0] += (a ? to_d(a[i]) : to_d(b[i])) * to_d(b[i]);
   block_partials<1>(v, partials);
 }
 
@@ -282,30 +272,27 @@ __global__ __launch_bounds__(kBlock) void k_finish_to(const double *__restrict__
   if (threadIdx.x == 0) *dst = take_sqrt ? sqrt(tot) : tot;
 }
 
-// k_mgs_step for j > 0 with the previous step's finish folded in: every block adds the previous
-// step's partials itself (finish_sum, the same sum as k_finish_to's) to get h(j-1, iv), block 0
-// stores it, then w = w - h(j-1) v_{j-1} and the partials of v_j . w (or w . w) go to partials.
-// The thread's first kMgsAhead elements of w, v_{j-1} and v_j are requested before the finish,
-// so their latency overlaps it; the elements are taken in the grid-stride order all the same.
+// Column 0 after a preconditioner that left the partials of v_0 . w: every block adds them itself
+// (finish_sum, the same sum in every block), block 0 stores h(0, 0), then w = w - h v_0 and the partials of
+// w . w.  The thread's first kMgsAhead elements are requested before the finish, so their latency overlaps it;
+// the elements are taken in the grid-stride order all the same.
 constexpr int kMgsAhead = 4;
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mgs_fold(T *__restrict__ w, const T *__restrict__ vprev,
-                                                     const T *__restrict__ vj, long long n,
-                                                     const double *__restrict__ pprev, int nprev, double *hprev,
+__global__ __launch_bounds__(kBlock) void k_mgs_fold(T *__restrict__ w, const T *__restrict__ v0, long long n,
+                                                     const double *__restrict__ pprev, int nprev, double *h00,
                                                      double *partials) {
   const long long i0 = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
   const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-  T wr[kMgsAhead], pr[kMgsAhead], jr[kMgsAhead];
+  T wr[kMgsAhead], pr[kMgsAhead];
 #pragma unroll
   for (int r = 0; r < kMgsAhead; ++r) {
     const long long i = i0 + r * stride;
     wr[r] = i < n ? w[i] : T(0);
-    pr[r] = i < n ? vprev[i] : T(0);
-    jr[r] = (vj && i < n) ? vj[i] : T(0);
+    pr[r] = i < n ? v0[i] : T(0);
   }
   const double h = finish_sum(pprev, nprev);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *hprev = h;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *h00 = h;
   const T a = static_cast<T>(-h);
   double v[1] = {0.0};
 #pragma unroll
@@ -314,15 +301,255 @@ __global__ __launch_bounds__(kBlock) void k_mgs_fold(T *__restrict__ w, const T 
     if (i < n) {
       const T wi = wr[r] + a * pr[r];
       w[i] = wi;
-      v[0] += vj ? to_d(jr[r]) * to_d(wi) : to_d(wi) * to_d(wi);
+      v[0] += to_d(wi) * to_d(wi);
     }
   }
   for (long long i = i0 + kMgsAhead * stride; i < n; i += stride) {
-    const T wi = w[i] + a * vprev[i];
+    const T wi = w[i] + a * v0[i];
     w[i] = wi;
-    v[0] += vj ? to_d(vj[i]) * to_d(wi) : to_d(wi) * to_d(wi);
+    v[0] += to_d(wi) * to_d(wi);
   }
   block_partials<1>(v, partials);
+}
+
+// ---- Gram-Schmidt of one Arnoldi column in two passes ------------------------------------------
+// Modified Gram-Schmidt takes h_j = v_j . (w - sum_{i<j} h_i v_i), one reduction after another.  With
+// a_j = v_j . w and l_ji = v_j . v_i (rounding-sized, not zero) that is h_j = a_j - sum_{i<j} h_i l_ji:
+// the same projections in exact arithmetic and with MGS's loss of orthogonality (Bjorck's triangular
+// form of MGS; Swirydowicz et al., "Low synchronization Gram-Schmidt and GMRES algorithms", 2021).  So one
+// pass over v_0 .. v_iv leaves the sums of all a_j and of the new row l_iv,j (k_gs_dots), and a second one
+// finishes them, solves the triangular system and subtracts (k_gs_update).  Dots and h are FP64; the
+// subtractions are those of MGS, in order, in the vectors' type.
+//   Bound: launch and load latency at these sizes (a basis vector of C24x30 is 0.8 MB).  Column iv took
+// iv + 1 launches of 5.0 us (FP64, C24x30) or 5.4 us (FP32, C48x50); it takes two, 5.4 + 7.9 us and 5.2 + 5.4 us:
+// FP64 GMRES(30) at C24x30 3.1 -> 0.95 ms, the mixed solve at C48x50 1.36 -> 1.16 ms.
+//   Shape: few enough blocks in the first pass that every block of the second can add all the partial
+// sums itself (at most 4096 doubles).  The second pass in blocks of 256 threads: 5.4 us (FP32, C48x50) where 512
+// and 1024 take 7.7.
+constexpr int kGsThreads = 1024, kGsUpd = 256, kGsBlocks = 256, kGsGroup = 8, kGsParts = 16;
+
+// Lane swaps of gfx950 halve what a lane holds: of two values a and b, lanes 0-31 (or the even rows of 16
+// lanes) are left with a's sum over the swapped halves and the others with b's.
+__device__ inline double swap_add(double a, double b, bool rows16) {
+  const unsigned alo = __double2loint(a), ahi = __double2hiint(a), blo = __double2loint(b), bhi = __double2hiint(b);
+  typedef unsigned U2 __attribute__((ext_vector_type(2)));
+  const U2 lo = rows16 ? __builtin_amdgcn_permlane16_swap(alo, blo, false, false)
+                       : __builtin_amdgcn_permlane32_swap(alo, blo, false, false);
+  const U2 hi = rows16 ? __builtin_amdgcn_permlane16_swap(ahi, bhi, false, false)
+                       : __builtin_amdgcn_permlane32_swap(ahi, bhi, false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+template <int CTRL>
+__device__ inline double dpp(double a) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ inline double sum8(double a) {  // over each 8 lanes
+  a += dpp<0xB1>(a);                       // quad_perm [1,0,3,2]
+  a += dpp<0x4E>(a);                       // quad_perm [2,3,0,1]
+  return a + dpp<0x141>(a);                // row_half_mirror
+}
+// v[0..15] summed over the wavefront: lane l gets the sums of values wave_sum16_value(l) (.x) and of the
+// next one (.y), 8 lanes alike.  17 additions in the vector ALU where a butterfly per value takes 96
+// through LDS.
+__device__ inline double2 wave_sum16(const double (&v)[16]) {
+  double a[8], b[4], c[2];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) a[q] = swap_add(v[q], v[q + 8], false);  // lanes >= 32: values 8..15
+#pragma unroll
+  for (int q = 0; q < 4; ++q) b[q] = swap_add(a[q], a[q + 4], true);   // odd rows: + 4
+  const bool up = (threadIdx.x & 8) != 0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // lanes 8-15 of a row: + 2
+    const double keep = up ? b[q + 2] : b[q], send = up ? b[q] : b[q + 2];
+    c[q] = keep + dpp<0x128>(send);  // row_ror:8
+  }
+  return make_double2(sum8(c[0]), sum8(c[1]));
+}
+__device__ inline int wave_sum16_value(int lane) {
+  return ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2;
+}
+
+// partials[block][q]: a_q = v_q . w for q <= iv, then l_iv,j = v_iv . v_j at q = iv + 1 + j.  Block row y
+// takes v_8y .. v_8y+7: the groups run side by side, since one after another each waits for its loads.
+template <typename T>
+__global__ __launch_bounds__(kGsThreads) void k_gs_dots(const T *__restrict__ V, const T *__restrict__ w, long long n,
+                                                        int iv, double *__restrict__ partials) {
+  __shared__ double s_p[kGsThreads / 64][2 * kGsGroup];
+  const int R = 2 * iv + 1, j0 = blockIdx.y * kGsGroup;
+  const long long stride = static_cast<long long>(gridDim.x) * kGsThreads;
+  const T *vl = V + static_cast<size_t>(iv) * n;
+  double v[2 * kGsGroup];
+#pragma unroll
+  for (int q = 0; q < 2 * kGsGroup; ++q) v[q] = 0.0;
+  const T *vq[kGsGroup];
+#pragma unroll
+  for (int q = 0; q < kGsGroup; ++q) vq[q] = V + static_cast<size_t>(min(j0 + q, iv)) * n;
+  auto add = [&](const T (&vj)[kGsGroup], T wv, T lv) {
+    const double wd = to_d(wv), ld = to_d(lv);
+#pragma unroll
+    for (int q = 0; q < kGsGroup; ++q) {
+      v[q] += to_d(vj[q]) * wd;
+      v[q + kGsGroup] += to_d(vj[q]) * ld;
+    }
+  };
+  long long i = static_cast<long long>(blockIdx.x) * kGsThreads + threadIdx.x;
+  for (; i + stride < n; i += 2 * stride) {
+    T x0[kGsGroup], x1[kGsGroup];
+#pragma unroll
+    for (int q = 0; q < kGsGroup; ++q) {
+      x0[q] = vq[q][i];
+      x1[q] = vq[q][i + stride];
+    }
+    const T w0 = w[i], w1 = w[i + stride], l0 = vl[i], l1 = vl[i + stride];
+    add(x0, w0, l0);
+    add(x1, w1, l1);
+  }
+  if (i < n) {
+    T x0[kGsGroup];
+#pragma unroll
+    for (int q = 0; q < kGsGroup; ++q) x0[q] = vq[q][i];
+    add(x0, w[i], vl[i]);
+  }
+  const double2 t = wave_sum16(v);
+  const int lane = threadIdx.x & 63;
+  if ((lane & 7) == 0) {
+    s_p[threadIdx.x >> 6][wave_sum16_value(lane)] = t.x;
+    s_p[threadIdx.x >> 6][wave_sum16_value(lane) + 1] = t.y;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 * kGsGroup) {
+    double s = 0.0;
+    for (int u = 0; u < kGsThreads / 64; ++u) s += s_p[u][threadIdx.x];
+    const int j = j0 + (threadIdx.x & (kGsGroup - 1));
+    const bool l = threadIdx.x >= kGsGroup;
+    if (l ? j < iv : j <= iv) partials[static_cast<size_t>(blockIdx.x) * R + (l ? iv + 1 + j : j)] = s;
+  }
+}
+
+// lanes that hold one block's sums in k_gs_update
+__host__ __device__ inline int gs_pad(int iv) { return iv < 8 ? 16 : iv < 16 ? 32 : iv < 32 ? 64 : 128; }
+// h(0..iv, iv) from the nb blocks' partials, in every block alike (block 0 stores h and the row of l),
+// then w -= sum_j h_j v_j, j in order, and the block's partial of w . w.  A thread's elements are VEC
+// neighbours (one load; n a multiple of VEC).
+template <typename T, int VEC>
+__global__ __launch_bounds__(kGsUpd) void k_gs_update(T *__restrict__ w, const T *__restrict__ V, long long n,
+                                                          int iv, int m, int nb, const double *__restrict__ pin,
+                                                          GmresState *st, double *__restrict__ partials) {
+  typedef T VT __attribute__((ext_vector_type(VEC)));
+  constexpr int kAhead = VEC * sizeof(T) == 16 ? kGsGroup : 2 * kGsGroup, kWaves = kGsUpd / 64;
+  __shared__ double s_l[kMaxKrylov * kMaxKrylov], s_sum[kWaves][2 * kMaxKrylov], s_tot[2 * kMaxKrylov];
+  __shared__ T s_h[kMaxKrylov];  // -h
+  const int R = 2 * iv + 1, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const long long nv = n / VEC, stride = static_cast<long long>(gridDim.x) * kGsUpd;
+  long long i = static_cast<long long>(blockIdx.x) * kGsUpd + tid;
+  auto wv = [&](long long k) { return reinterpret_cast<VT *>(w) + k; };
+  auto vv = [&](int q, long long k) { return *(reinterpret_cast<const VT *>(V + static_cast<size_t>(q) * n) + k); };
+  // the thread's first elements of w and of the first kAhead vectors, the partials and the rows of l, requested
+  // together
+  VT wi = i < nv ? *wv(i) : VT{}, va[kAhead];
+#pragma unroll
+  for (int q = 0; q < kAhead; ++q) va[q] = (i < nv && q <= iv) ? vv(q, i) : VT{};
+  // partials: pad lanes per block of k_gs_dots, so a thread adds nb * pad / kGsUpd of them (at most kGsParts,
+  // gs_blocks), then the threads of one sum in a wavefront, then the wavefronts
+  const int pad = gs_pad(iv);
+  double s = 0.0;
+  {
+    const int q = tid & (pad - 1), parts = kGsUpd / pad, b0 = tid / pad;
+    double t[kGsParts];
+#pragma unroll
+    for (int u = 0; u < kGsParts; ++u)
+      t[u] = (q < R && b0 + u * parts < nb) ? pin[static_cast<size_t>(b0 + u * parts) * R + q] : 0.0;
+    for (int k0 = tid; k0 < iv * kMaxKrylov; k0 += 8 * kGsUpd) {
+      double lk[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) lk[u] = k0 + u * kGsUpd < iv * kMaxKrylov ? st->l[k0 + u * kGsUpd] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (k0 + u * kGsUpd < iv * kMaxKrylov) s_l[k0 + u * kGsUpd] = lk[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kGsParts; ++u) s += t[u];
+    if (pad <= 32) s += __shfl_xor(s, 32, 64);
+    if (pad == 16) s += __shfl_xor(s, 16, 64);
+    // a wavefront holds sums 0..63 (the second of a pair 64..127 when pad is 128)
+    if (lane < pad) s_sum[wid][(pad == 128 ? (wid & 1) * 64 : 0) + lane] = s;
+  }
+  __syncthreads();
+  if (tid < R) {
+    double t = 0.0;
+    const int step = pad == 128 ? 2 : 1, u0 = pad == 128 ? tid >> 6 : 0;
+#pragma unroll
+    for (int u = 0; u < kWaves; ++u) t += u * step + u0 < kWaves ? s_sum[(u * step + u0) & (kWaves - 1)][tid] : 0.0;
+    s_tot[tid] = t;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    double a = tid <= iv ? s_tot[tid] : 0.0;
+    for (int c0 = 0; c0 < iv; c0 += 8) {
+      double lc[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int c = min(c0 + u, iv - 1);
+        lc[u] = tid < iv ? s_l[c * kMaxKrylov + tid] : s_tot[iv + 1 + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int c = c0 + u;
+        if (c < iv) {
+          const double hc = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), c),
+                                             __builtin_amdgcn_readlane(__double2loint(a), c));
+          if (tid > c && tid <= iv) a -= hc * lc[u];
+        }
+      }
+    }
+    if (tid <= iv) s_h[tid] = static_cast<T>(-a);
+    if (blockIdx.x == 0) {
+      if (tid <= iv) st->h[static_cast<size_t>(iv) * (m + 1) + tid] = a;
+      if (tid < iv) st->l[tid * kMaxKrylov + iv] = s_tot[iv + 1 + tid];
+    }
+  }
+  __syncthreads();
+  double v[1] = {0.0};
+  while (i < nv) {
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+      if (q <= iv) wi = wi + s_h[q] * va[q];
+    for (int j = kAhead; j <= iv; j += kGsGroup) {
+      VT vj[kGsGroup];
+#pragma unroll
+      for (int q = 0; q < kGsGroup; ++q) vj[q] = vv(min(j + q, iv), i);
+#pragma unroll
+      for (int q = 0; q < kGsGroup; ++q)
+        if (j + q <= iv) wi = wi + s_h[j + q] * vj[q];
+    }
+    *wv(i) = wi;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[0] += to_d(wi[e]) * to_d(wi[e]);
+    i += stride;
+    if (i < nv) {
+      wi = *wv(i);
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) va[q] = q <= iv ? vv(q, i) : VT{};
+    }
+  }
+  wave_sum<1>(v);
+  if (lane == 0) s_sum[wid][0] = v[0];
+  __syncthreads();
+  if (tid == 0) {
+    double t = 0.0;
+#pragma unroll
+    for (int u = 0; u < kWaves; ++u) t += s_sum[u][0];
+    partials[blockIdx.x] = t;
+  }
+}
+
+// block columns of k_gs_dots: its groups of 8 vectors share kGsBlocks blocks, and a thread of
+// k_gs_update adds at most kGsParts partials
+inline int gs_blocks(long long n, int iv) {
+  const int groups = (iv + kGsGroup) / kGsGroup;
+  return grid_for(n, kGsThreads, std::min(std::max(1, kGsBlocks / groups), kGsParts * kGsUpd / gs_pad(iv)));
 }
 
 // The Givens rotations of sci_iterative_solver_mod.f90:929-953 (k_givens below) formed one
@@ -587,6 +814,7 @@ static void *g_gm[6] = {nullptr};
 static size_t g_gm_bytes[6] = {0};
 static GmresState *g_gstate = nullptr;
 static double *g_gpart = nullptr;
+static double *g_gdots = nullptr;  // k_gs_dots' partials
 static double *g_host_scalar = nullptr;
 static hipEvent_t g_gev[2] = {nullptr, nullptr};  // the inner solve's per-column residual reads
 constexpr int kGmBlocks = 1024;
@@ -609,6 +837,8 @@ static int gm_init() {
     if (int rc = dmalloc(reinterpret_cast<void **>(&g_gstate), sizeof(GmresState))) return rc;
   if (!g_gpart)
     if (int rc = dmalloc(reinterpret_cast<void **>(&g_gpart), sizeof(double) * 2 * kGmBlocks)) return rc;
+  if (!g_gdots)
+    if (int rc = dmalloc(reinterpret_cast<void **>(&g_gdots), sizeof(double) * 2 * kMaxKrylov * kGsBlocks)) return rc;
   if (!g_host_scalar)
     LF_HIP(hipHostMalloc(reinterpret_cast<void **>(&g_host_scalar), sizeof(double) * 4, hipHostMallocDefault));
   for (auto &e : g_gev)
@@ -616,44 +846,46 @@ static int gm_init() {
   return LFRIC_OK;
 }
 
-// The Gram-Schmidt steps j = 0 .. iv+1 of Arnoldi column iv (w against v_0 .. v_iv, then
-// ||w||), and v_{iv+1} = w / h(iv+1, iv) unless iv is the cycle's last column.  Each step's
-// partial sums are finished by the next kernel's blocks themselves (partials in two alternating
-// halves of the scratch), so a step is one launch; the h values are those of separate
-// finishing kernels bit for bit.
-// first_parts > 0: step 0's partials (v_0 . w) are already in the first half of the scratch,
-// that many of them (left there by the preconditioner's apply).
+// Gram-Schmidt of Arnoldi column iv (w against v_0 .. v_iv, then ||w||), and v_{iv+1} = w /
+// h(iv+1, iv) unless iv is the cycle's last column.  Column 0 after a preconditioner that left its
+// partial sums (first_parts of v_0 . w in the scratch) takes one pass, the others two (k_gs_dots,
+// k_gs_update); the next kernel's blocks finish ||w||^2 themselves.
 template <typename T>
-static int arnoldi_mgs(T *w, T *V, long long n, int iv, int m, double *h, GmresState *gst = nullptr,
-                       int first = 0, int first_parts = 0) {
-  const int vg = grid_for(n);
-  double *part[2] = {g_gpart, g_gpart + kGmBlocks};
-  if (!first_parts)
-    LAUNCHK(k_mgs_step<T>, kGmBlocks, kBlock, w, static_cast<const T *>(nullptr), static_cast<const T *>(V), n,
-            static_cast<const double *>(nullptr), part[0]);
-  for (int j = 1; j <= iv + 1; ++j) {
-    const T *vj = j <= iv ? V + static_cast<size_t>(j) * n : nullptr;
-    const int nprev = (j == 1 && first_parts) ? first_parts : kGmBlocks;
-    LAUNCHK(k_mgs_fold<T>, kGmBlocks, kBlock, w, V + static_cast<size_t>(j - 1) * n, vj, n, part[(j - 1) & 1],
-            nprev, &h[iv * (m + 1) + (j - 1)], part[j & 1]);
+static int arnoldi_column(T *w, T *V, long long n, int iv, int m, GmresState *st, bool givens, int first = 0,
+                          int first_parts = 0) {
+  double *part = g_gpart + kGmBlocks;
+  int np = kGmBlocks;
+  if (iv == 0 && first_parts) {
+    LAUNCHK(k_mgs_fold<T>, kGmBlocks, kBlock, w, V, n, g_gpart, first_parts, &st->h[0], part);
+  } else {
+    const int nb = gs_blocks(n, iv);
+    LAUNCHK(k_gs_dots<T>, dim3(nb, (iv + kGsGroup) / kGsGroup), kGsThreads, V, w, n, iv, g_gdots);
+    // 16-byte elements where the vectors are long enough to fill the GPU with them: a thread then has
+    // one round of loads instead of two or three
+    constexpr int kVec = 16 / sizeof(T);
+    const bool vec = n % kVec == 0 && n / kVec >= 128 * kGsThreads;
+    np = grid_for(vec ? n / kVec : n, kGsUpd, kGsBlocks * kGsThreads / kGsUpd);
+    if (vec)
+      LAUNCHK((k_gs_update<T, kVec>), np, kGsUpd, w, V, n, iv, m, nb, g_gdots, st, part);
+    else
+      LAUNCHK((k_gs_update<T, 1>), np, kGsUpd, w, V, n, iv, m, nb, g_gdots, st, part);
   }
-  double *hlast = &h[iv * (m + 1) + iv + 1];
+  double *hlast = &st->h[static_cast<size_t>(iv) * (m + 1) + iv + 1];
   if (iv < m - 1)
-    LAUNCHK(k_scale_fold<T>, std::min(vg, kGmBlocks), kBlock, V + static_cast<size_t>(iv + 1) * n, w, n,
-            part[(iv + 1) & 1], kGmBlocks, hlast, gst, iv, m, first);
-  else if (gst)
-    LAUNCHK(k_finish_givens, 1, kBlock, part[(iv + 1) & 1], kGmBlocks, hlast, gst, iv, m, first);
+    LAUNCHK(k_scale_fold<T>, std::min(grid_for(n), kGmBlocks), kBlock, V + static_cast<size_t>(iv + 1) * n, w, n, part,
+            np, hlast, givens ? st : nullptr, iv, m, first);
+  else if (givens)
+    LAUNCHK(k_finish_givens, 1, kBlock, part, np, hlast, st, iv, m, first);
   else
-    LAUNCHK(k_finish_to, 1, kBlock, part[(iv + 1) & 1], kGmBlocks, hlast, 1);
+    LAUNCHK(k_finish_to, 1, kBlock, part, np, hlast, 1);
   LF_HIP(hipGetLastError());
   return LFRIC_OK;
 }
 
-// ||v||^2 or v.w into *dst (device) with the fused MGS kernel
+// a.b (sq: ||b||) into *dst (device)
 template <typename T>
-static int dot_into(const T *a, T *b, long long n, double *dst, bool sq) {
-  LAUNCHK(k_mgs_step<T>, kGmBlocks, kBlock, b, static_cast<const T *>(nullptr), sq ? static_cast<const T *>(nullptr) : a,
-          n, static_cast<const double *>(nullptr), g_gpart);
+static int dot_into(const T *a, const T *b, long long n, double *dst, bool sq) {
+  LAUNCHK(k_dot_partials<T>, kGmBlocks, kBlock, sq ? static_cast<const T *>(nullptr) : a, b, n, g_gpart);
   LAUNCHK(k_finish_to, 1, kBlock, g_gpart, kGmBlocks, dst, sq ? 1 : 0);
   LF_HIP(hipGetLastError());
   return LFRIC_OK;
@@ -718,8 +950,7 @@ static int gmres_t(const lfric_linop *A, const lfric_prec *P, T *x, const T *b, 
     if (int rc = prec_apply_any(P, prec, r, s, n)) return rc;
     // beta = ||s|| and v_0 = s / beta: the partials of s . s, then one kernel that finishes them
     // (as k_finish_to) and scales (as k_scale_by_inv)
-    LAUNCHK(k_mgs_step<T>, kGmBlocks, kBlock, s, static_cast<const T *>(nullptr), static_cast<const T *>(nullptr), n,
-            static_cast<const double *>(nullptr), g_gpart);
+    LAUNCHK(k_dot_partials<T>, kGmBlocks, kBlock, static_cast<const T *>(nullptr), s, n, g_gpart);
     LAUNCHK(k_scale_fold<T>, std::min(grid_for(n), kGmBlocks), kBlock, V, s, n, g_gpart, kGmBlocks, &st->beta,
             static_cast<GmresState *>(nullptr), 0, m, 0);
     int k = m;  // columns made in this cycle
@@ -729,16 +960,16 @@ static int gmres_t(const lfric_linop *A, const lfric_prec *P, T *x, const T *b, 
       if (!P || P->kind == 0) {  // identity: w = P^-1 (A v_iv) is the apply's output itself
         if (int rc = linop_apply(A, viv, w)) return rc;
       } else if (coltri_tiles(P) > 0 && coltri_tiles(P) <= kGmBlocks) {
-        // the tiled column block-Jacobi also leaves Gram-Schmidt step 0's partials (v_0 . w)
+        // the tiled column block-Jacobi also leaves column 0's partials (v_0 . w)
         if (int rc = linop_apply(A, viv, s)) return rc;
-        if (int rc = prec_apply_impl(P, prec, s, w, n, V, g_gpart)) return rc;
-        first_parts = coltri_tiles(P);
+        if (int rc = prec_apply_impl(P, prec, s, w, n, iv == 0 ? V : nullptr, g_gpart)) return rc;
+        first_parts = iv == 0 ? coltri_tiles(P) : 0;
       } else {
         if (int rc = linop_apply(A, viv, s)) return rc;  // s = A w (w = v_iv)
         if (int rc = prec_apply_any(P, prec, s, w, n)) return rc;  // w = P^-1 s
       }
       // Gram-Schmidt and Givens column iv
-      if (int rc = arnoldi_mgs<T>(w, V, n, iv, m, st->h, st, cyc == 1 ? 1 : 0, first_parts)) return rc;
+      if (int rc = arnoldi_column<T>(w, V, n, iv, m, st, true, cyc == 1 ? 1 : 0, first_parts)) return rc;
       if (early && iv < m - 1) {
         double *slot = g_host_scalar + 2 + (iv & 1);
         LF_HIP(hipMemcpyAsync(slot, &st->ratio, sizeof(double), hipMemcpyDeviceToHost, cur_stream()));
@@ -826,7 +1057,7 @@ static int fgmres_t(const lfric_linop *A, const lfric_prec *P, T *x, const T *b,
       T *viv = V + static_cast<size_t>(iv) * n, *pviv = PV + static_cast<size_t>(iv) * n;
       if (int rc = prec_apply_any(P, prec, viv, pviv, n)) return rc;  // Pv = P^-1 v
       if (int rc = linop_apply(A, pviv, w)) return rc;               // w = s = A Pv
-      if (int rc = arnoldi_mgs<T>(w, V, n, iv, m, st->h)) return rc;
+      if (int rc = arnoldi_column<T>(w, V, n, iv, m, st, false)) return rc;
     }
     LAUNCHK(k_givens, 1, 64, st, m);
     LAUNCHK(k_gmres_update<T>, vg, kBlock, dx, PV, n, m, st->u);  // dx += sum u_iv Pv_iv
