@@ -57,6 +57,8 @@ FunctionSpace::~FunctionSpace() {
   dfree(d_goff, goff_bytes);
   dfree(d_gent, gent_bytes);
   dfree(d_w0tab, w0tab_bytes);
+  dfree(d_w2tab, w2tab_bytes);
+  dfree(d_w2col, w2col_bytes);
 }
 
 // Scratch vectors of the solvers, kept between solves (grown on demand).  Slots: 0-2 CG's r, z,
@@ -302,9 +304,7 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
   if (a.x_zero) {
     if (int rc = launch_copy(a.prec, r, a.b, a.n)) return rc;
   } else {
-    if (int rc = launch_lma_apply_solver(a.A, a.x, r, nullptr)) return rc;
-    if (a.bc)
-      if (int rc = launch_enforce_bc(*a.A->to, a.prec, r, nullptr)) return rc;
+    if (int rc = a.bc ? launch_lma_apply_bc(a.A, a.x, r, nullptr) : launch_lma_apply_solver(a.A, a.x, r, nullptr)) return rc;
     if (int rc = launch_cg_residual(a.prec, r, a.b, a.n)) return rc;
   }
   if (int rc = launch_cg_init_norm(a.prec, r, a.n, g_state)) return rc;
@@ -337,9 +337,9 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
       if (fused) {
         if (int rc = launch_lma_apply_gather_dot(a.A, p, z, pz_partials, &g_state->done)) return rc;
       } else {
-        if (int rc = launch_lma_apply_solver(a.A, p, z, &g_state->done)) return rc;
-        if (a.bc)
-          if (int rc = launch_enforce_bc(*a.A->to, a.prec, z, &g_state->done)) return rc;
+        if (int rc = a.bc ? launch_lma_apply_bc(a.A, p, z, &g_state->done)
+                          : launch_lma_apply_solver(a.A, p, z, &g_state->done))
+          return rc;
         if (int rc = launch_cg_dot_pz(a.prec, p, z, a.n, g_state, c.d_partials)) return rc;
       }
       if (!fold)
@@ -741,13 +741,17 @@ int lfric_op_create(const lfric_fs *to, const lfric_fs *from, int precision, lfr
     return rc;
   }
   LF_HIP(hipMemsetAsync(op->d, 0, op->bytes, cur_stream()));
-  // the table of the lowest-order W0 apply, here so that the apply itself never allocates (it may be
-  // captured)
+  // the tables of the lowest-order W0 and W2 applies and of the W2 transpose, here so that the applies
+  // themselves never allocate (they may be captured)
+  int rc = LFRIC_OK;
   if (op->to == op->from)
-    if (int rc = build_w0_table(*op->to)) {
-      lfric_op_destroy(op);
-      return rc;
-    }
+    rc = t.ndf == 8 ? build_w0_table(*op->to) : build_w2_table(*op->to, true);
+  else if (t.ndf == 1 && t.top_mask == 0)
+    rc = build_w2_table(*op->from, false);
+  if (rc) {
+    lfric_op_destroy(op);
+    return rc;
+  }
   *out = op;
   return LFRIC_OK;
 }

@@ -115,6 +115,15 @@ struct FunctionSpace {
   void *d_w0tab = nullptr;
   int w0tab_cols = 0;
   size_t w0tab_bytes = 0;
+  // lowest-order W2 spaces whose side faces have at most two cells: each cell's neighbours
+  // (w2_apply.hip); null otherwise
+  std::vector<int4> w2_nbr;
+  void *d_w2tab = nullptr;
+  size_t w2tab_bytes = 0;
+  // and their dof columns' cells, for square operators
+  void *d_w2col = nullptr;
+  int w2_ncols = 0;
+  size_t w2col_bytes = 0;
   ~FunctionSpace();
 };
 
@@ -212,18 +221,13 @@ struct lfric_linop {
   std::shared_ptr<lfric::FunctionSpace> space;  // domain and range
   void *t_w2 = nullptr, *t_w3 = nullptr;      // scratch of the composite apply
   size_t t_w2_bytes = 0, t_w3_bytes = 0;
-  mutable int fused = -1;  // kind 1: the two-kernel composite applies (set on first use)
-  mutable int hcol_state = 0;  // kind 1: 1 the W2 column table is built, -1 the mesh does not allow one
-  mutable void *d_hcol = nullptr;
+  mutable int fused = -1;  // kind 1: the fused composite applies (set on first use)
+  mutable int hcol_state = 0;  // kind 1: 1 the one-kernel apply's tables are built, -1 the mesh does not allow it
+  mutable void *d_hcol = nullptr;  // each cell's side neighbours' W3 column bases, -1 where there is none
   mutable size_t hcol_bytes = 0;
-  // kind 1: D's entries in transpose-gather order (two per W2 dof) and the D version they hold
-  mutable void *d_dtc = nullptr;
-  mutable size_t dtc_bytes = 0;
-  mutable unsigned long long dtc_version = ~0ull;
-  // kind 1: D's rows and M3 compacted in the divergence kernel's thread order, and the D and
-  // M3 versions they hold
-  mutable void *d_drc = nullptr;
-  mutable size_t drc_bytes = 0;
-  mutable unsigned long long drc_dver = ~0ull, drc_mver = ~0ull;
+  // kind 1: D and M3 in the kernel's thread order, and the D and M3 versions they hold
+  mutable void *d_helm = nullptr;
+  mutable size_t helm_bytes = 0;
+  mutable unsigned long long helm_dver = ~0ull, helm_mver = ~0ull;
   ~lfric_linop();
 };

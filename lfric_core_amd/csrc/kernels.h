@@ -68,6 +68,8 @@ int launch_build_rows(lfric_op *op);
 int launch_lma_apply_gather_marked(const lfric_op *op, const void *x, void *y, hipEvent_t mark, bool *two_phase);
 // the apply form the solvers use (lfric_set_apply_form)
 int launch_lma_apply_solver(const lfric_op *op, const void *x, void *y, const int *skip);
+// the same, then enforce_bc on y, in one kernel where the space allows it
+int launch_lma_apply_bc(const lfric_op *op, const void *x, void *y, const int *skip);
 int launch_lma_apply_mrhs(const lfric_op *op, const void *x, void *y, int nrhs, int variant);
 int launch_op_invert_local(const lfric_op *A, lfric_op *Ainv);
 int launch_build_sym(lfric_op *op, int levels_per_thread);
@@ -89,7 +91,18 @@ bool mfma_apply_supported(const lfric_op *op);
 // per thread with register-staged x (order-1 W0), 0 none (gather form)
 int batch_colour_form(const lfric_op *op);
 int launch_lma_transpose(const lfric_op *op, const void *x, void *y);
-// the Helmholtz composite in two kernels (lowest-order W3 <- W2), equal to the chain of
+// Each cell's side neighbours of a lowest-order W2 space, and (columns) the cells of its dof columns: no table,
+// with LFRIC_OK, for other spaces and where a side face has more than two cells.  Over them: the apply of a
+// square operator, with the gather form's sums or (colour) the colour-ordered form's, bit for bit, and enforce_bc
+// with bc; the transpose of a 1 x 6 operator (both always faster than the kernels without tables, which stay
+// for other spaces); and the Helmholtz composite in one kernel: build_helm_table sets hcol_state, 1 where
+// launch_helm applies; w2_apply.hip
+int build_w2_table(FunctionSpace &f, bool columns);
+int launch_w2_gather(const lfric_op *op, const void *x, void *y, bool colour, double *partials, const int *skip, int bc);
+int launch_transpose_w2(const lfric_op *op, const void *x, void *y);
+int build_helm_table(const lfric_linop *L);
+int launch_helm(const lfric_linop *L, const void *x, void *y);
+// the Helmholtz composite in one kernel or two (lowest-order W3 <- W2), equal to the chain of
 // transpose, division, divergence, M3 apply and axpy bit for bit; helmholtz_fusable says
 // whether it applies to the operator
 bool helmholtz_fusable(const lfric_linop *L);

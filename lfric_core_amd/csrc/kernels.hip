@@ -1251,7 +1251,7 @@ __global__ __launch_bounds__(kBlock) void k_transpose_colour(const T *__restrict
 }
 
 // ---- Helmholtz composite y = M3 x + tau D diag(M2)^-1 D^T x in two kernels ------------------
-// (W3 <- W2 lowest order: D holds 1 x 6 per element, M3 1 x 1.)  The first is the transpose in
+// For meshes without the neighbour table of the one-kernel form (w2_apply.hip).  (W3 <- W2 lowest order: D holds 1 x 6 per element, M3 1 x 1.)  The first is the transpose in
 // gather form with the division by m2 folded in: W2 dof (column, level m) adds its cells'
 // contributions in colour order, the first written and the rest added, each the colour-
 // ordered transpose's chain (row of layer m, then the top partner's of layer m-1), then divides
@@ -1286,70 +1286,6 @@ __global__ __launch_bounds__(kBlock) void k_helm_transpose_div(const T *__restri
   t[d] = total / m2[d];
 }
 
-// The composite's copy of D in transpose-gather order.  A table built for the composite holds
-// each W2 column's (at most two) cells as one int4, {ebase, W3 dof * 8 + face} per cell in
-// the column's colour order (the second ebase -1 when the column has one cell); the W2 lowest-
-// order roles are fixed (face 4 the bottom, its partner the top face 5).  Per W2 dof (column,
-// level m) the copy holds the two entries of D that its row of D^T takes (a side face: the
-// column's first and second cell at layer m; a bottom/top face column: the bottom face at
-// layer m and the top face at layer m-1), zero where there is none, so the transpose reads one
-// coalesced pair per dof instead of one value out of each cell's 16-byte chunk of faces, and
-// one level of dependent index loads where the gather lists take three.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_build_dtc(const T *__restrict__ D, size_t gs, const int2 *__restrict__ cols,
-                                                     const int4 *__restrict__ tab, int ncols, int nl,
-                                                     T *__restrict__ out) {
-  const int H = nl + 1;
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= ncols * H) return;
-  const int col = p / H, m = p - col * H;
-  const int2 ci = cols[col];
-  if (m == nl && !ci.y) return;
-  const int4 c = tab[col];
-  T a = T(0), b = T(0);
-  if ((c.y & 7) == 4) {
-    if (m < nl) a = D[aidx<T>(gs, static_cast<long long>(c.x) + m, 4)];
-    if (m > 0) b = D[aidx<T>(gs, static_cast<long long>(c.x) + m - 1, 5)];
-  } else {
-    a = D[aidx<T>(gs, static_cast<long long>(c.x) + m, c.y & 7)];
-    if (c.z >= 0) b = D[aidx<T>(gs, static_cast<long long>(c.z) + m, c.w & 7)];
-  }
-  const size_t d = static_cast<size_t>(ci.x) + m;
-  out[2 * d] = a;
-  out[2 * d + 1] = b;
-}
-
-// k_helm_transpose_div over that copy and the table: the same terms in the same order, bit for
-// bit
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_helm_transpose_div_dtc(const T *__restrict__ dtc,
-                                                                  const T *__restrict__ x3, const T *__restrict__ m2,
-                                                                  T *__restrict__ t, const int2 *__restrict__ cols,
-                                                                  const int4 *__restrict__ tab, int ncols, int nl) {
-  using T2 = typename std::conditional<sizeof(T) == 8, double2, float2>::type;
-  const int H = nl + 1;
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= ncols * H) return;
-  const int col = p / H, m = p - col * H;
-  const int2 ci = cols[col];
-  if (m == nl && !ci.y) return;
-  const int4 c = tab[col];
-  const size_t d = static_cast<size_t>(ci.x) + m;
-  const T2 v = reinterpret_cast<const T2 *>(dtc)[d];
-  const int b3 = c.y >> 3;
-  T total;
-  if ((c.y & 7) == 4) {
-    T acc = T(0);
-    if (m < nl) acc = fma(v.x, x3[b3 + m], acc);
-    if (m > 0) acc = fma(v.y, x3[b3 + m - 1], acc);
-    total = acc;
-  } else {
-    total = fma(v.x, x3[b3 + m], T(0));
-    if (c.z >= 0) total = total + fma(v.y, x3[(c.w >> 3) + m], T(0));
-  }
-  t[d] = total / m2[d];
-}
-
 // the second: per W3 dof (cell, layer m) the divergence row (k_lma_colour's chain over the 6
 // faces), M3's 1 x 1 product and y = M3 x + tau (D t) as k_axpy forms it
 template <typename T>
@@ -1368,43 +1304,6 @@ __global__ __launch_bounds__(kBlock) void k_helm_dg_m3(const T *__restrict__ D, 
   for (int j = 0; j < 6; ++j) acc = fma(D[aidx<T>(gsd, e, j)], t[b2[j] + m], acc);
   const size_t d = static_cast<size_t>(map3[pos]) + m;
   const T y3 = fma(M3[aidx<T>(gs3, e, 0)], x3[d], T(0));
-  y[d] = y3 + tau * acc;
-}
-
-// The composite's compact copy of D's rows and M3 in k_helm_dg_m3's thread order u = pos * nl
-// + m: row j < 6 of D at out[j * nu + u], M3 at out[6 * nu + u].  The element layout pads a
-// 1 x 6 element to two 16-byte chunks and a 1 x 1 element to one (each thread of the apply then
-// pulls whole chunks for one value); the copy holds the values alone, coalesced per entry.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_build_drc(const T *__restrict__ D, size_t gsd, const T *__restrict__ M3,
-                                                     size_t gs3, const int *__restrict__ ebase, int ncells, int nl,
-                                                     T *__restrict__ out) {
-  const int nu = ncells * nl;
-  const int u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= nu) return;
-  const int pos = u / nl, m = u - pos * nl;
-  const long long e = static_cast<long long>(ebase[pos]) + m;
-#pragma unroll
-  for (int j = 0; j < 6; ++j) out[static_cast<size_t>(j) * nu + u] = D[aidx<T>(gsd, e, j)];
-  out[static_cast<size_t>(6) * nu + u] = M3[aidx<T>(gs3, e, 0)];
-}
-
-// k_helm_dg_m3 over that copy: the same products in the same order, bit for bit
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_helm_dg_m3_drc(const T *__restrict__ drc, const T *__restrict__ t,
-                                                          const int *__restrict__ map2, const T *__restrict__ x3,
-                                                          const int *__restrict__ map3, T *__restrict__ y, int ncells,
-                                                          int nl, T tau) {
-  const int nu = ncells * nl;
-  const int u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= nu) return;
-  const int pos = u / nl, m = u - pos * nl;
-  const int *b2 = map2 + static_cast<size_t>(pos) * 6;
-  T acc = T(0);
-#pragma unroll
-  for (int j = 0; j < 6; ++j) acc = fma(drc[static_cast<size_t>(j) * nu + u], t[b2[j] + m], acc);
-  const size_t d = static_cast<size_t>(map3[pos]) + m;
-  const T y3 = fma(drc[static_cast<size_t>(6) * nu + u], x3[d], T(0));
   y[d] = y3 + tau * acc;
 }
 
@@ -2272,6 +2171,7 @@ static int apply_colours_t(const lfric_op *op, const T *x, T *y, const int *d_sk
   RoleKind rk = role_kind(to);
   if (rk == RoleKind::W0K1 && from.ndf == 27) return launch_colour_rows27(op, x, y, 1, d_skip);
   if (to.d_w0tab && op->to == op->from) return launch_w0_gather(op, x, y, true, nullptr, d_skip);
+  if (to.d_w2col && op->to == op->from) return launch_w2_gather(op, x, y, true, nullptr, d_skip, 0);
   const size_t S = op->gs;
   const int nl = to.nlayers;
   for (int c = 0; c < to.ncolours; ++c) {
@@ -2481,6 +2381,12 @@ static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gathe
     }
     if (to.d_w0tab && op->to == op->from) {
       (void)launch_w0_gather(op, x, y, false, ex.partials, ex.skip);
+      return;
+    }
+  }
+  if constexpr (N2 == 6 && std::is_same<R, RolesW2K0>::value) {
+    if (to.d_w2col && op->to == op->from) {
+      (void)launch_w2_gather(op, x, y, false, ex.partials, ex.skip, 0);
       return;
     }
   }
@@ -2783,6 +2689,15 @@ int launch_lma_apply_solver(const lfric_op *op, const void *x, void *y, const in
   return ctx().apply_form == 1 ? gather_any(op, x, y, GatherExtra{nullptr, skip}) : launch_lma_apply(op, x, y, skip);
 }
 
+int launch_lma_apply_bc(const lfric_op *op, const void *x, void *y, const int *skip) {
+  const FunctionSpace &f = *op->to;
+  // the bottom and top faces' flags are those that the W2 apply over its table can enforce itself
+  if (ctx().apply_form == 1 && f.d_w2col && op->to == op->from && f.bc_bottom == (1u << 4) && f.bc_top == (1u << 5))
+    return launch_w2_gather(op, x, y, false, nullptr, skip, 1);
+  if (int rc = launch_lma_apply_solver(op, x, y, skip)) return rc;
+  return launch_enforce_bc(f, op->precision, y, skip);
+}
+
 int launch_gather_blocks(const lfric_op *op, int *nblocks) {
   if (int rc = build_gather(*op->to)) return rc;
   *nblocks = gather_dot_blocks(op);
@@ -2817,6 +2732,9 @@ static int transpose_t(const lfric_op *op, const T *x, T *y) {
 }
 
 int launch_lma_transpose(const lfric_op *op, const void *x, void *y) {
+  if (op->to->ndf == 1 && op->to->top_mask == 0 && op->from->d_w2tab &&
+      (op->precision == LFRIC_R64 || op->precision == LFRIC_R32))
+    return launch_transpose_w2(op, x, y);
   if (op->precision == LFRIC_R64)
     return transpose_t<double>(op, static_cast<const double *>(x), static_cast<double *>(y));
   if (op->precision == LFRIC_R32)
@@ -3140,94 +3058,25 @@ bool helmholtz_fusable(const lfric_linop *L) {
          w2.ebase == w3.ebase && (L->precision == LFRIC_R64 || L->precision == LFRIC_R32);
 }
 
-// the composite's column table for k_build_dtc and k_helm_transpose_div_dtc (the gather lists
-// of the W2 space resolved to ebase and W3 dof per cell); none when a column has more than two
-// cells
-static int build_helm_table(const lfric_linop *L) {
-  if (L->hcol_state) return LFRIC_OK;
-  const FunctionSpace &w2 = *L->D->from, &w3 = *L->D->to;
-  struct Item {
-    int base, pos, df;
-  };
-  std::vector<Item> items;
-  for (int p = 0; p < w2.ncells; ++p)
-    for (int d = 0; d < 6; ++d)
-      if (!((w2.top_mask >> d) & 1u)) items.push_back({w2.dofmap[static_cast<size_t>(w2.cell_of_pos[p]) * 6 + d] - 1, p, d});
-  std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.base < b.base; });
-  std::vector<int4> tab;
-  bool ok = true;
-  for (size_t q = 0; q < items.size() && ok; ++q) {
-    const Item &it = items[q];
-    const int ent = w2.ebase[it.pos], bj = (w3.dofmap[w3.cell_of_pos[it.pos]] - 1) * 8 + it.df;
-    if (q == 0 || it.base != items[q - 1].base) {
-      tab.push_back(make_int4(ent, bj, -1, 0));
-    } else if (tab.back().z < 0) {
-      tab.back().z = ent;
-      tab.back().w = bj;
-    } else {
-      ok = false;
-    }
-  }
-  ok = ok && static_cast<int>(tab.size()) == w2.gather_ncols && static_cast<long long>(w3.undf) * 8 < (1LL << 31) &&
-       static_cast<long long>(w2.gather_ncols) * (w2.nlayers + 1) + kBlock < (1LL << 31);
-  L->hcol_state = -1;
-  if (!ok) return LFRIC_OK;
-  L->hcol_bytes = sizeof(int4) * tab.size();
-  if (int rc = dmalloc(reinterpret_cast<void **>(&L->d_hcol), L->hcol_bytes)) return rc;
-  LF_HIP(hipMemcpy(L->d_hcol, tab.data(), L->hcol_bytes, hipMemcpyHostToDevice));
-  L->hcol_state = 1;
-  return LFRIC_OK;
-}
-
 template <typename T>
 static int helmholtz_t(const lfric_linop *L, const T *x, T *y) {
   FunctionSpace &w2 = *L->D->from;
   const FunctionSpace &w3 = *L->D->to;
   if (int rc = build_gather(w2)) return rc;
-  if (int rc = build_helm_table(L)) return rc;
   T *t = static_cast<T *>(L->t_w2);
-  const int tgrid = grid_for(static_cast<long long>(w2.gather_ncols) * (w2.nlayers + 1));
-  if (L->hcol_state == 1 && L->dtc_version != L->D->version) {  // (re)build the copy of D
-    if (!L->d_dtc) {
-      L->dtc_bytes = 2 * sizeof(T) * static_cast<size_t>(w2.undf);
-      if (int rc = dmalloc(&L->d_dtc, L->dtc_bytes)) return rc;
-    }
-    LAUNCH((k_build_dtc<T>), tgrid, static_cast<const T *>(L->D->d), L->D->gs, w2.d_gcol,
-           static_cast<const int4 *>(L->d_hcol), w2.gather_ncols, w2.nlayers, static_cast<T *>(L->d_dtc));
-    CHECK_LAUNCH();
-    L->dtc_version = L->D->version;
-  }
-  if (L->hcol_state == 1)
-    LAUNCH((k_helm_transpose_div_dtc<T>), tgrid, static_cast<const T *>(L->d_dtc), x,
-           static_cast<const T *>(L->m2->d), t, w2.d_gcol, static_cast<const int4 *>(L->d_hcol), w2.gather_ncols,
-           w2.nlayers);
-  else
-    LAUNCH((k_helm_transpose_div<T>), tgrid, static_cast<const T *>(L->D->d), L->D->gs, w3.d_ebase, x, w3.d_map,
-           static_cast<const T *>(L->m2->d), t, w2.d_gcol, w2.d_goff, w2.d_gent, w2.gather_ncols, w2.nlayers,
-           roles_of(w2));
-  const int ugrid = grid_for(static_cast<long long>(w3.ncells) * w3.nlayers);
-  if (L->hcol_state == 1 && (L->drc_dver != L->D->version || L->drc_mver != L->M3->version)) {
-    if (!L->d_drc) {  // (re)build the compact rows of D and M3
-      L->drc_bytes = 7 * sizeof(T) * static_cast<size_t>(w3.ncells) * w3.nlayers;
-      if (int rc = dmalloc(&L->d_drc, L->drc_bytes)) return rc;
-    }
-    LAUNCH((k_build_drc<T>), ugrid, static_cast<const T *>(L->D->d), L->D->gs, static_cast<const T *>(L->M3->d),
-           L->M3->gs, w3.d_ebase, w3.ncells, w3.nlayers, static_cast<T *>(L->d_drc));
-    CHECK_LAUNCH();
-    L->drc_dver = L->D->version;
-    L->drc_mver = L->M3->version;
-  }
-  if (L->hcol_state == 1)
-    LAUNCH((k_helm_dg_m3_drc<T>), ugrid, static_cast<const T *>(L->d_drc), t, w2.d_map, x, w3.d_map, y, w3.ncells,
-           w3.nlayers, static_cast<T>(L->tau));
-  else
-    LAUNCH((k_helm_dg_m3<T>), ugrid, static_cast<const T *>(L->D->d), L->D->gs, static_cast<const T *>(L->M3->d),
-           L->M3->gs, w3.d_ebase, t, w2.d_map, x, w3.d_map, y, w3.ncells, w3.nlayers, static_cast<T>(L->tau));
+  LAUNCH((k_helm_transpose_div<T>), grid_for(static_cast<long long>(w2.gather_ncols) * (w2.nlayers + 1)),
+         static_cast<const T *>(L->D->d), L->D->gs, w3.d_ebase, x, w3.d_map, static_cast<const T *>(L->m2->d), t,
+         w2.d_gcol, w2.d_goff, w2.d_gent, w2.gather_ncols, w2.nlayers, roles_of(w2));
+  LAUNCH((k_helm_dg_m3<T>), grid_for(static_cast<long long>(w3.ncells) * w3.nlayers),
+         static_cast<const T *>(L->D->d), L->D->gs, static_cast<const T *>(L->M3->d), L->M3->gs, w3.d_ebase, t, w2.d_map,
+         x, w3.d_map, y, w3.ncells, w3.nlayers, static_cast<T>(L->tau));
   CHECK_LAUNCH();
   return LFRIC_OK;
 }
 
 int launch_helmholtz_fused(const lfric_linop *L, const void *x, void *y) {
+  if (int rc = build_helm_table(L)) return rc;
+  if (L->hcol_state == 1) return launch_helm(L, x, y);
   if (L->precision == LFRIC_R64)
     return helmholtz_t<double>(L, static_cast<const double *>(x), static_cast<double *>(y));
   return helmholtz_t<float>(L, static_cast<const float *>(x), static_cast<float *>(y));

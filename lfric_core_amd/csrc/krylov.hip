@@ -734,8 +734,7 @@ static size_t esz(int p) { return p == LFRIC_R64 ? 8 : p == LFRIC_R32 ? 4 : 2; }
 
 int linop_apply(const lfric_linop *L, const void *x, void *y) {
   if (L->kind == 0) {
-    if (int rc = launch_lma_apply_solver(L->A, x, y, nullptr)) return rc;
-    return L->apply_bc ? launch_enforce_bc(*L->space, L->precision, y, nullptr) : LFRIC_OK;
+    return L->apply_bc ? launch_lma_apply_bc(L->A, x, y, nullptr) : launch_lma_apply_solver(L->A, x, y, nullptr);
   }
   // y = M3 x + tau * D (D^T x / m2)
   if (L->fused < 0) L->fused = helmholtz_fusable(L) ? 1 : 0;
@@ -1094,8 +1093,7 @@ lfric_prec::~lfric_prec() {
 
 lfric_linop::~lfric_linop() {
   dfree(d_hcol, hcol_bytes);
-  dfree(d_dtc, dtc_bytes);
-  dfree(d_drc, drc_bytes);
+  dfree(d_helm, helm_bytes);
   dfree(t_w2, t_w2_bytes);
   dfree(t_w3, t_w3_bytes);
 }
@@ -1137,6 +1135,11 @@ int lfric_linop_create_helmholtz(const lfric_op *M3, const lfric_op *D, const lf
   L->tau = tau;
   L->precision = D->precision;
   L->space = M3->to;
+  // the one-kernel apply over the W2 space's neighbour table needs no scratch
+  if (D->from->d_w2tab && helmholtz_fusable(L)) {
+    *out = L;
+    return LFRIC_OK;
+  }
   L->t_w2_bytes = esz(L->precision) * static_cast<size_t>(D->from->undf);
   L->t_w3_bytes = esz(L->precision) * static_cast<size_t>(M3->to->undf);
   if (int rc = dmalloc(&L->t_w2, L->t_w2_bytes)) {
