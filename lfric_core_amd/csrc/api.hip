@@ -64,12 +64,12 @@ FunctionSpace::~FunctionSpace() {
 // Scratch vectors of the solvers, kept between solves (grown on demand).  Slots: 0-2 CG's r, z,
 // p; 3 the true-residual vector; 4 CG's p.Ap partials; 5, 6 and 8 the refinement driver's FP32
 // right-hand side, FP32 correction and FP64 residual (live across its inner CG solves); 7 host
-// staging.
+// staging; 9, 10 the small CG's q and second p.
 struct Workspace {
   void *p = nullptr;
   size_t bytes = 0;
 };
-static Workspace g_ws[9];
+static Workspace g_ws[11];
 static SolverState *g_state = nullptr;
 static SolverState *g_state_host = nullptr;
 
@@ -269,13 +269,17 @@ struct CgArgs {
 // then reads the device state once; kernels of iterations past convergence return at once.
 // Byte offsets of r, z, p and the p.Ap partials inside the allocation-free CG's scratch array:
 // each piece starts on a 256-byte boundary.  Returns the bytes used.
-static size_t cg_scratch_layout(size_t vb, int pz_blocks, size_t off[4]) {
+// The small CG's q and second p follow them (it takes vectors of at most 1.5 MB, so they fit).
+static size_t cg_scratch_layout(size_t vb, int pz_blocks, size_t off[6]) {
   const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   off[0] = 0;
   off[1] = up(vb);
   off[2] = off[1] + up(vb);
   off[3] = off[2] + up(vb);
-  return off[3] + up(sizeof(double) * static_cast<size_t>(std::max(pz_blocks, 1)));
+  const size_t end = off[3] + up(sizeof(double) * static_cast<size_t>(std::max(pz_blocks, 1)));
+  off[4] = end;
+  off[5] = end + up(vb);
+  return end;
 }
 
 // scratch_base: null for the grown workspace slots; else the device address of the
@@ -284,7 +288,7 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
   Context &c = ctx();
   const size_t vb = esize(a.prec) * static_cast<size_t>(a.n);
   void *r, *z, *p;
-  size_t soff[4] = {0, 0, 0, 0};
+  size_t soff[6] = {0, 0, 0, 0, 0, 0};
   if (scratch_base) {
     cg_scratch_layout(vb, 1, soff);
     r = scratch_base + soff[0];
@@ -331,6 +335,27 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
   const int npz = fused ? pz_blocks : kRedBlocks;
   const bool fold = npz <= kFoldMaxPartials;
   const bool sym = fused && cg_sym_usable(a.A);
+  if (fused && !sym && cg_w0_usable(a.A)) {
+    void *v[6] = {a.x, r, z, nullptr, p, nullptr};
+    if (scratch_base) {
+      cg_scratch_layout(vb, pz_blocks, soff);
+      v[3] = scratch_base + soff[4];
+      v[5] = scratch_base + soff[5];
+    } else {
+      if (int rc = ws_get(9, vb, &v[3])) return rc;
+      if (int rc = ws_get(10, vb, &v[5])) return rc;
+    }
+    for (int ch = 0, k = 0; ch < max_chunks; ++ch) {
+      for (int i = 0; i < every; ++i, ++k)
+        if (int rc = launch_cg_w0_iteration(a.A, v, a.diag, g_state, k)) return rc;
+      if (int rc = launch_cg_w0_test(a.A, g_state, k)) return rc;
+      LF_HIP(hipMemcpyAsync(g_state_host, g_state, sizeof(SolverState), hipMemcpyDeviceToHost, cur_stream()));
+      LF_HIP(hipStreamSynchronize(cur_stream()));
+      if (g_state_host->done) break;
+    }
+    out = *g_state_host;
+    return LFRIC_OK;
+  }
   long long it = 0;  // iterations enqueued: their parity picks the rz slot
   for (int ch = 0; ch < max_chunks; ++ch) {
     for (int i = 0; i < every; ++i, ++it) {
@@ -1232,7 +1257,7 @@ int lfric_cg_solve_noalloc(const lfric_op *A, const lfric_prec *P, lfric_vec *x,
   LF_CHECK(base, LFRIC_E_STATE, "cg_solve_noalloc: no scratch address recorded for this device");
   const bool fused = ctx().apply_form == 1;
   const bool listed = A->to->d_gcol != nullptr;
-  size_t off[4];
+  size_t off[6];
   const size_t need = cg_scratch_layout(esize(A->precision) * static_cast<size_t>(x->n),
                                         fused && listed ? gather_dot_blocks(A) : 1, off);
   LF_CHECK(need <= kScratchBytes, LFRIC_E_UNSUPPORTED,

@@ -9,24 +9,12 @@
 #include "internal.h"
 #include "kernels.h"
 #include "role_kind.h"
+#include "w0_table.h"
 
 namespace lfric {
 namespace {
 
-// Table entry of a dof column (W0Col in int4 units): the element slot bases of its cells in colour
-// order, its base dof with the cell count and each cell's bottom row, and each cell's 4 bottom
-// vertex columns (the top vertices lie one level up in the same columns).
-struct W0Col {
-  int4 ebase;   // of cell 0..3
-  int4 head;    // base dof, cells, row of cell 0..3 (one byte each), 0
-  int4 xcol[4];
-};
-static_assert(sizeof(W0Col) == 96, "W0Col is read as 6 int4");
-
-// Thread (column, level m).  COLOUR: each cell's bottom row of layer m and top row of layer m-1 are
-// two chains from zero and their sum is added, as k_lma_colour does (the same bits); else one chain
-// runs through the cells, as in k_lma_gather.  The roles of a W0 space put a cell's top vertex j+4 one
-// level above its bottom vertex j, so its two rows' x are 4 columns at 3 levels, each loaded once.
+// Thread (column, level m): w0_point.
 //   Bound: HBM on large meshes, the chain of dependent loads on small ones.  The column's cells, rows
 // and vertex columns come with one round of loads where the lists take three (offsets, entries, map),
 // and there is one launch where the colours take four that each re-read x and y.  FP64 / FP32,
@@ -39,8 +27,6 @@ __global__ __launch_bounds__(kBlock) void k_w0_gather(const T *__restrict__ A, s
                                                       T *__restrict__ y, int ncols, int nl, double *partials,
                                                       const int *skip, int xwin) {
   if (skip && *skip) return;
-  constexpr int V = chunk_entries<T>(), NC = 8 / V;
-  typedef T VecT __attribute__((ext_vector_type(V)));
   const int H = nl + 1;
   const int lb = xcd_block(blockIdx.x, gridDim.x, xwin);
   const unsigned t = static_cast<unsigned>(lb) * kBlock + threadIdx.x;
@@ -48,58 +34,8 @@ __global__ __launch_bounds__(kBlock) void k_w0_gather(const T *__restrict__ A, s
   const unsigned col = valid ? t / H : 0;
   const int m = valid ? static_cast<int>(t - col * H) : 0;
   const W0Col *tc = tab + col;
-  const int4 eb4 = tc->ebase, head = tc->head;
-  int4 xc[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) xc[k] = tc->xcol[k];
-  const int eb[4] = {eb4.x, eb4.y, eb4.z, eb4.w};
-  const int cnt = valid ? head.y : 0;
-  const bool has_m = m < nl, has_p = m > 0;
-  T acc = T(0);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= cnt) break;
-    const int i = (head.z >> (8 * k)) & 255;
-    const long long e = static_cast<long long>(eb[k]) + m;
-    const T *Ae = A + static_cast<size_t>(e >> 6) * gs + static_cast<size_t>(e & 63) * V;
-    const T *rt = Ae + static_cast<size_t>(i + 4) * NC * 64 * V, *rb = Ae + static_cast<size_t>(i) * NC * 64 * V;
-    VecT top[NC], bot[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      top[c] = has_p ? *reinterpret_cast<const VecT *>(rt + static_cast<size_t>(c) * 64 * V) : VecT{};
-      bot[c] = has_m ? *reinterpret_cast<const VecT *>(rb + static_cast<size_t>(c) * 64 * V) : VecT{};
-    }
-    const int b[4] = {xc[k].x, xc[k].y, xc[k].z, xc[k].w};
-    T xl[3][4];  // x of the cell's 4 columns at levels m-1, m, m+1
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      xl[0][j] = has_p ? x[b[j] + m - 1] : T(0);
-      xl[1][j] = x[b[j] + m];
-      xl[2][j] = has_m ? x[b[j] + m + 1] : T(0);
-    }
-    if constexpr (COLOUR) {
-      T c = T(0), cp = T(0);
-      if (has_m) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) c = fma(bot[j / V][j % V], j < 4 ? xl[1][j] : xl[2][j - 4], c);
-      }
-      if (has_p) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) cp = fma(top[j / V][j % V], j < 4 ? xl[0][j] : xl[1][j - 4], cp);
-      }
-      const T out = c + cp;
-      acc = k == 0 ? out : acc + out;
-    } else {
-      if (has_p) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc = fma(top[j / V][j % V], j < 4 ? xl[0][j] : xl[1][j - 4], acc);
-      }
-      if (has_m) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc = fma(bot[j / V][j % V], j < 4 ? xl[1][j] : xl[2][j - 4], acc);
-      }
-    }
-  }
+  const int4 head = tc->head;
+  const T acc = w0_point<T, COLOUR>(A, gs, tc, head, valid ? head.y : 0, m, nl, [&](int d) { return x[d]; });
   if (valid) y[static_cast<size_t>(head.x) + m] = acc;
   if constexpr (DOT) {
     double v[1] = {valid ? to_d(acc) * to_d(x[static_cast<size_t>(head.x) + m]) : 0.0};

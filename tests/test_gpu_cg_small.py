@@ -1,0 +1,53 @@
+"""Conjugate gradients in two kernels an iteration (small lowest-order W0 problems) against the form over the
+colour-ordered apply in separate kernels, whose sums run in another order: the same iterates up to rounding
+after a fixed number of iterations (the recurrences' error grows by the condition of B B^T + 0.1 I elements, below
+100: 1e4 eps of the norm), counts within one to a tolerance, and the ends of a solve.  Sizes of one block,
+several, a partial one, and both sides of the largest it takes (1.5 MB vectors)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _cg(hip, op, b, P, form, **kw):
+    hip.set_apply_form(form)
+    try:
+        x = hip.FieldVector(op.fs_to, P)
+        x.set_scalar(0.0)
+        res = hip.ConjugateGradient(op, hip.DiagonalPreconditioner.from_operator(op), **kw).apply(x, b)
+        return res, x.export_field()
+    finally:
+        hip.set_apply_form(1)
+
+
+@pytest.mark.parametrize("prec", ["R64", "R32"])
+@pytest.mark.parametrize("n,nl", [(2, 2), (3, 4), (5, 7), (12, 20), (25, 48), (25, 49), (32, 60)])
+def test_two_kernel_iteration(hip, n, nl, prec):
+    P, eps = (hip.R64, np.finfo(np.float64).eps) if prec == "R64" else (hip.R32, np.finfo(np.float32).eps)
+    fs = hip.FunctionSpace.cubedsphere(n, nl)
+    op = hip.LmaOperator(fs).generate_spd(n + nl)
+    op = op if P == hip.R64 else op.convert(P)
+    b = hip.FieldVector(fs, P).fill_uniform(n, 3)
+    for iters in (1, 2, 6):
+        kw = dict(r_tol=1e-30, a_tol=0.0, max_iter=iters, monitor_convergence=False, check_every=4)
+        (r1, x1), (r0, x0) = (_cg(hip, op, b, P, form, **kw) for form in (1, 0))
+        assert r1.iterations == r0.iterations == iters
+        assert np.linalg.norm(x1 - x0) <= 1e4 * eps * np.linalg.norm(x0)
+    kw = dict(r_tol=1e-8 if P == hip.R64 else 1e-4, a_tol=0.0, max_iter=100, check_every=8)
+    (r1, x1), (r0, x0) = (_cg(hip, op, b, P, form, **kw) for form in (1, 0))
+    assert r1.status == r0.status == 0 and abs(r1.iterations - r0.iterations) <= 1
+
+
+def test_ends_of_a_solve(hip):
+    fs = hip.FunctionSpace.cubedsphere(6, 9)
+    op = hip.LmaOperator(fs).generate_spd(1)
+    zero = hip.FieldVector(fs)
+    zero.set_scalar(0.0)
+    res, x = _cg(hip, op, zero, hip.R64, 1, r_tol=1e-10, a_tol=0.0, max_iter=50)
+    assert res.status == 0 and res.iterations == 0 and not x.any()
+    bad = hip.FieldVector(fs).import_field(np.full(fs.undf, np.nan))
+    with pytest.raises(hip.LfricError):
+        _cg(hip, op, bad, hip.R64, 1, r_tol=1e-10, a_tol=0.0, max_iter=50)
+    b = hip.FieldVector(fs).fill_uniform(1, 3)
+    res, _ = _cg(hip, op, b, hip.R64, 1, r_tol=1e-12, a_tol=0.0, max_iter=3)
+    assert res.status == 1 and res.iterations == 3
