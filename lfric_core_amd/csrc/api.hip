@@ -34,6 +34,10 @@ int dmalloc(void **p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 64;
   hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && batch_buffers_release()) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return fail(LFRIC_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));

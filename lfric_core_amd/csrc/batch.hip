@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <vector>
 
@@ -610,13 +611,51 @@ namespace {
 
 constexpr double kEps = 2.220446049250313e-16;
 
+// Device buffers of destroyed batches and removed problems, kept for the next of the same size: a program
+// that solves one batch after another spent 4 of 23 ms (8 problems) in hipMalloc and hipFree.  At most 1 GiB in
+// all (kept buffers count as free, not as held by live handles), given back when an allocation of the library
+// fails (batch_buffers_release).  Only idle buffers are put: their owners wait for the device first.
+std::mutex g_buf_mu;
+std::vector<std::pair<void *, size_t>> g_buf;
+size_t g_buf_bytes = 0;
+constexpr size_t kBufMax = size_t{1} << 30;
+
+int buf_get(void **p, size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lk(g_buf_mu);
+    for (size_t i = 0; i < g_buf.size(); ++i)
+      if (g_buf[i].second == bytes) {
+        *p = g_buf[i].first;
+        g_buf.erase(g_buf.begin() + static_cast<long>(i));
+        g_buf_bytes -= bytes;
+        ctx().bytes += static_cast<long long>(bytes);
+        return LFRIC_OK;
+      }
+  }
+  return dmalloc(p, bytes);
+}
+
+void buf_put(void *p, size_t bytes) {
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> lk(g_buf_mu);
+    if (bytes > 0 && g_buf_bytes + bytes <= kBufMax) {
+      g_buf.emplace_back(p, bytes);
+      g_buf_bytes += bytes;
+      ctx().bytes -= static_cast<long long>(bytes);
+      return;
+    }
+  }
+  dfree(p, bytes);
+}
+
 int ensure(void **p, size_t &cap, size_t need, size_t elem) {
   if (need <= cap && *p) return LFRIC_OK;
   dfree(*p, cap * elem);
   *p = nullptr;
   cap = 0;
   const size_t c = std::max<size_t>(need, 16) * 2;
-  if (int rc = dmalloc(p, c * elem)) return rc;
+  if (int rc = buf_get(p, c * elem)) return rc;
   cap = c;
   return LFRIC_OK;
 }
@@ -680,7 +719,7 @@ int alloc_state(lfric_batch &B, int nr, int *scal0) {
   if (need > B.cap_state) {
     const size_t cap = std::max<size_t>(need * 2, 64);
     RhsDev *d = nullptr, *h = nullptr;
-    if (int rc = dmalloc(reinterpret_cast<void **>(&d), cap * sizeof(RhsDev))) return rc;
+    if (int rc = buf_get(reinterpret_cast<void **>(&d), cap * sizeof(RhsDev))) return rc;
     if (hipHostMalloc(reinterpret_cast<void **>(&h), cap * sizeof(RhsDev), hipHostMallocDefault) != hipSuccess) {
       dfree(d, cap * sizeof(RhsDev));
       return fail(LFRIC_E_NOMEM, "pinned host state");
@@ -709,7 +748,7 @@ int rebuild(lfric_batch &B) {
   for (Problem *p : B.active)
     if (apply_form(B, *p) == kFormSym27 && !p->zs) {
       const size_t need = sizeof(float) * s27_zalloc(p->A32->to->ncells, p->A32->to->nlayers, p->nrhs);
-      if (int rc = dmalloc(reinterpret_cast<void **>(&p->zs), need)) return rc;
+      if (int rc = buf_get(reinterpret_cast<void **>(&p->zs), need)) return rc;
       p->zs_bytes = need;
     }
   // order-1 problems first (their own apply kernel), then the gather-form and matrix-core groups,
@@ -1095,9 +1134,9 @@ int refine_all(lfric_batch &B, const std::vector<Problem *> &ps) {
 }
 
 void free_problem(lfric_batch &B, Problem &p) {
-  dfree(p.d, p.bytes32);
-  dfree(p.r64, p.bytes64);
-  dfree(p.zs, p.zs_bytes);
+  buf_put(p.d, p.bytes32);
+  buf_put(p.r64, p.bytes64);
+  buf_put(p.zs, p.zs_bytes);
   p.d = nullptr;
   p.r64 = nullptr;
   p.zs = nullptr;
@@ -1147,6 +1186,18 @@ int run_rounds(lfric_batch &B, int rounds, int *nactive) {
 }
 
 }  // namespace
+
+bool batch_buffers_release() {
+  std::vector<std::pair<void *, size_t>> all;
+  {
+    std::lock_guard<std::mutex> lk(g_buf_mu);
+    all.swap(g_buf);
+    g_buf_bytes = 0;
+  }
+  for (auto &b : all) (void)hipFree(b.first);
+  return !all.empty();
+}
+
 }  // namespace lfric
 
 using namespace lfric;
@@ -1200,8 +1251,8 @@ int lfric_batch_add(lfric_batch *B, const lfric_op *A64, const lfric_op *A32, co
   p->bytes32 = sizeof(float) * static_cast<size_t>(p->n) * 4;
   p->bytes64 = sizeof(double) * static_cast<size_t>(p->n);
   p->scal0 = -1;
-  if (int rc = dmalloc(reinterpret_cast<void **>(&p->d), p->bytes32)) return rc;
-  if (int rc = dmalloc(reinterpret_cast<void **>(&p->r64), p->bytes64)) {
+  if (int rc = buf_get(reinterpret_cast<void **>(&p->d), p->bytes32)) return rc;
+  if (int rc = buf_get(reinterpret_cast<void **>(&p->r64), p->bytes64)) {
     free_problem(*B, *p);
     return rc;
   }
@@ -1278,7 +1329,7 @@ int lfric_batch_remove(lfric_batch *B, int id) {
   for (size_t i = 0; i < B->probs.size(); ++i)
     if (B->probs[i]->id == id) {
       if (B->probs[i]->inner_running) B->dirty = true;
-      LF_HIP(hipStreamSynchronize(cur_stream()));
+      LF_HIP(hipDeviceSynchronize());  // as in lfric_batch_destroy
       free_problem(*B, *B->probs[i]);
       B->probs.erase(B->probs.begin() + static_cast<long>(i));
       return LFRIC_OK;
@@ -1351,18 +1402,18 @@ int lfric_batch_stats(const lfric_batch *B, long long *iterations, int *block, i
 
 void lfric_batch_destroy(lfric_batch *B) {
   if (!B) return;
-  (void)hipStreamSynchronize(cur_stream());
+  (void)hipDeviceSynchronize();  // the buffers go to the next batch idle, whatever stream it uses
   for (auto &u : B->probs) free_problem(*B, *u);
   drop_graph(*B);
-  dfree(B->d_state, B->cap_state * sizeof(RhsDev));
+  buf_put(B->d_state, B->cap_state * sizeof(RhsDev));
   if (B->h_state) (void)hipHostFree(B->h_state);
-  dfree(B->d_desc, B->cap_desc * sizeof(ProbDev));
-  dfree(B->d_tile0, B->cap_tile0 * sizeof(int));
-  dfree(B->d_vtile0, B->cap_vtile0 * sizeof(int));
-  dfree(B->d_partials, B->cap_partials * sizeof(double));
+  buf_put(B->d_desc, B->cap_desc * sizeof(ProbDev));
+  buf_put(B->d_tile0, B->cap_tile0 * sizeof(int));
+  buf_put(B->d_vtile0, B->cap_vtile0 * sizeof(int));
+  buf_put(B->d_partials, B->cap_partials * sizeof(double));
   dfree(B->d_scratch, sizeof(double) * kSlot * B->scratch_slots);
   dfree(B->d_counter, sizeof(unsigned int) * kCounters);
-  dfree(B->d_ctile0, B->cap_ctile0 * sizeof(int));
+  buf_put(B->d_ctile0, B->cap_ctile0 * sizeof(int));
   if (B->h_scratch) (void)hipHostFree(B->h_scratch);
   delete B;
 }

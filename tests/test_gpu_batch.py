@@ -132,3 +132,26 @@ def test_batch_copy_forms_equal_colour_and_gather_forms(hip, orc):
         same = col if order == 1 else gat
         np.testing.assert_array_equal(cop[i][0], same[i][0])
         assert [r.iterations for r in cop[i][1]] == [r.iterations for r in same[i][1]]
+
+
+def test_batches_one_after_another_reuse_their_buffers(hip):
+    """A second batch of the same problems, after the first is destroyed, gets the first one's buffers: the
+    same results bit for bit (nothing is read before it is written), and no device memory is held by
+    either afterwards."""
+    from lfric_core_amd.batch import Batch, build_problem
+    probs = [build_problem(4, 5, 0, 4, 1), build_problem(3, 4, 1, 2, 2), build_problem(5, 3, 1, 1, 3)]
+    held, out = [hip.device_bytes()], []
+    for _ in range(3):
+        bt = Batch(r_tol=1e-8, a_tol=0.0, max_iter=500, check_every=8)
+        for p in probs:
+            p["x"].set_scalar(0.0)
+            bt.add(p["op64"], p["op32"], p["d32"], p["x"], p["b"])
+        bt.solve()
+        bt.close()
+        held.append(hip.device_bytes())
+        out.append([p["x"].export_field() for p in probs])
+    # the first batch may build its operators' lists; after it nothing grows
+    assert held[1] == held[2] == held[3]
+    for later in out[1:]:
+        for a, b in zip(out[0], later):
+            np.testing.assert_array_equal(a, b)
