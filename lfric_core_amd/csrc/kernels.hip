@@ -1049,7 +1049,9 @@ __device__ inline double sym_gather_point(long long t, const T *__restrict__ z, 
   return to_d(acc) * to_d(x[static_cast<size_t>(ci.x) + m]);
 }
 
-// one point per thread
+// kSymPoints points per thread, kBlock apart: over the int4 table all their loads are requested before any
+// is added (C96x70 FP32: 21.3 us a point at a time, 15.6 us).
+constexpr int kSymPoints = 4;
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_sym_gather(const T *__restrict__ z, const T *__restrict__ x,
                                                         T *__restrict__ y, const int2 *__restrict__ cols,
@@ -1057,8 +1059,44 @@ __global__ __launch_bounds__(kBlock) void k_sym_gather(const T *__restrict__ z, 
                                                         const int4 *__restrict__ zu, int ncols, int nl, const int *skip,
                                                         int xwin) {
   if (skip && *skip) return;
-  const long long t = static_cast<long long>(xcd_block(blockIdx.x, gridDim.x, xwin)) * kBlock + threadIdx.x;
-  (void)sym_gather_point<T>(t, z, x, y, cols, off, ent, zu, ncols, nl);
+  const long long t0 = static_cast<long long>(xcd_block(blockIdx.x, gridDim.x, xwin)) * kBlock * kSymPoints + threadIdx.x;
+  const unsigned H = nl + 1;
+  const long long total = static_cast<long long>(ncols) * H;
+  if (!zu || total >= (1LL << 31)) {
+    for (int e = 0; e < kSymPoints; ++e)
+      (void)sym_gather_point<T>(t0 + e * kBlock, z, x, y, cols, off, ent, zu, ncols, nl);
+    return;
+  }
+  T v[kSymPoints][4];
+  int4 us[kSymPoints];
+  int2 ci[kSymPoints];
+  unsigned m[kSymPoints];
+  bool ok[kSymPoints];
+#pragma unroll
+  for (int e = 0; e < kSymPoints; ++e) {
+    const long long t = t0 + e * kBlock;
+    ok[e] = t < total;
+    const unsigned col = ok[e] ? static_cast<unsigned>(t) / H : 0;
+    m[e] = ok[e] ? static_cast<unsigned>(t) - col * H : 0;
+    us[e] = zu[col];
+    ci[e] = cols[col];
+  }
+#pragma unroll
+  for (int e = 0; e < kSymPoints; ++e) {
+    ok[e] = ok[e] && (m[e] < H - 1 || ci[e].y);
+    const int w[4] = {us[e].x, us[e].y, us[e].z, us[e].w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[e][q] = ok[e] && w[q] >= 0 ? z[static_cast<size_t>(w[q]) * H + m[e]] : T(0);
+  }
+#pragma unroll
+  for (int e = 0; e < kSymPoints; ++e) {
+    const int w[4] = {us[e].x, us[e].y, us[e].z, us[e].w};
+    T acc = v[e][0];
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+      if (w[q] >= 0) acc = acc + v[e][q];
+    if (ok[e]) y[static_cast<size_t>(ci[e].x) + m[e]] = acc;
+  }
 }
 
 // with the x.y partial sums of the CG's p.(A p): a fixed grid of kRedBlocks blocks walks the
@@ -2305,7 +2343,9 @@ static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gathe
         LAUNCH((k_sym_gather_dot<T>), kRedBlocks, static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff,
                to.d_gent, op->d_symzu, to.gather_ncols, to.nlayers, ex.partials, ex.skip, op->xwin);
       else
-        LAUNCH((k_sym_gather<T>), grid, static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent,
+        LAUNCH((k_sym_gather<T>),
+               grid_for(static_cast<long long>(to.gather_ncols) * (to.nlayers + 1), kBlock * kSymPoints),
+               static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent,
                op->d_symzu, to.gather_ncols, to.nlayers, ex.skip, op->xwin);
       return;
     }
