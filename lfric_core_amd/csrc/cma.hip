@@ -212,13 +212,13 @@ __global__ __launch_bounds__(kBlock) void k_cma_appinv(const T *__restrict__ C, 
   }
 }
 
-// LDS-staged forms for columns of up to kMaxStagedRows rows.  A block is one wavefront of 64
-// columns.  The fields are column-contiguous (a column's dofs are consecutive), so reading them
-// one lane per column touches 64 cache lines per instruction; instead the block copies its 64
-// columns of x into LDS with lanes running along each column (64 consecutive values per
-// instruction), the lanes then work one column each out of LDS, and the result goes back to
-// HBM the same way.  Each column's slice is padded to an odd stride S so that lane c's row r,
-// at c*S + r, falls in a different bank for every lane.  The arithmetic is unchanged.
+// LDS-staged forms for columns of up to kMaxStagedRows rows.  A block takes 64 columns.  The fields are
+// column-contiguous (a column's dofs are consecutive), so reading them one lane per column touches
+// 64 cache lines per instruction; instead the block copies its 64 columns of x into LDS with lanes
+// running along each column (64 consecutive values per instruction), the lanes then work one
+// column each out of LDS, and the result goes back to HBM the same way.  Each column's slice is
+// padded to an odd stride S so that lane c's row r, at c*S + r, falls in a different bank for every
+// lane.  The arithmetic is unchanged.
 constexpr int kColBlock = 64;
 constexpr int kMaxStagedRows = 127;
 // dynamic LDS one block may use: the device's per-block limit, read once
@@ -235,152 +235,185 @@ size_t max_block_lds() {
 
 __host__ __device__ inline int staged_stride(int n) { return n | 1; }
 
-// Each lane loads the base dof of one column and the offsets of rows lane and lane + 64 once;
-// the bases are then broadcast by lane shuffles, and the loads of kStageBatch columns are all
-// issued before any of them is written to LDS, so a block waits for memory 64 / kStageBatch
-// times.  n <= 2 * kColBlock.
+// One wave copies columns cfirst..clast-1 of the block's ncol between x and LDS; mybase is the base dof
+// of column `lane` of the block, n <= 2 * kColBlock - 1.  With about one wave on a SIMD the copy is
+// bound by the instructions it issues, not by its bytes.  So the first 64 rows take a column an
+// instruction, its base read into a scalar register (one vector instruction beside the load, where a
+// shuffled base needed the address of every lane), and the remaining n % 64 rows take as many whole
+// columns an instruction as fit 64 lanes (C96x70 FP32: 7 instructions instead of 64 of six lanes each).
+// kStageBatch (kRestBatch) instructions' loads are requested before any is used; a load past the block's last
+// column repeats that column, so that none of them needs a branch.
 constexpr int kStageBatch = 16;
+constexpr int kRestBatch = 8;
 
-template <typename T, int B = kStageBatch>
-__device__ inline void stage_columns_in(T *__restrict__ xs, int S, const T *__restrict__ x,
-                                        const int *__restrict__ map, int ndf, const int *__restrict__ ind,
-                                        int n, int pos0, int nc, int cfirst = 0, int clast = kColBlock) {
+template <typename T>
+__device__ inline void stage_columns_in(T *__restrict__ xs, int S, const T *__restrict__ x, int mybase,
+                                        const int *__restrict__ ind, int n, int ncol, int cfirst, int clast) {
   const int lane = threadIdx.x & (kColBlock - 1);
-  const int mybase = pos0 + lane < nc ? map[static_cast<size_t>(pos0 + lane) * ndf] : 0;
-  const int r0 = lane, r1 = lane + kColBlock;
-  const int o0 = r0 < n ? ind[r0] : 0, o1 = r1 < n ? ind[r1] : 0;
-  const int ncol = min(kColBlock, nc - pos0);
-  for (int c0 = cfirst; c0 < clast; c0 += B) {
-    T v0[B], v1[B];
+  const int full = n >= kColBlock ? kColBlock : 0, rest = n - full;
+  if (full) {
+    const long long o = ind[lane];
+#pragma unroll 1
+    for (int c0 = cfirst; c0 < clast; c0 += kStageBatch) {
+      T v[kStageBatch];
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int base = __shfl(mybase, c0 + u, kColBlock);
-      const bool ok = c0 + u < ncol;
-      v0[u] = ok && r0 < n ? x[static_cast<size_t>(base) + o0] : T(0);
-      v1[u] = ok && r1 < n ? x[static_cast<size_t>(base) + o1] : T(0);
+      for (int u = 0; u < kStageBatch; ++u)
+        v[u] = (x + __builtin_amdgcn_readlane(mybase, min(c0 + u, ncol - 1)))[o];
+#pragma unroll
+      for (int u = 0; u < kStageBatch; ++u)
+        if (c0 + u < clast) xs[(c0 + u) * S + lane] = v[u];
     }
+  }
+  if (rest) {
+    const int per = kColBlock / rest, cl = lane / rest, r = full + (cl < per ? lane - cl * rest : 0);
+    const long long o = ind[r];
+#pragma unroll 1
+    for (int c0 = cfirst; c0 < clast; c0 += kRestBatch * per) {
+      T v[kRestBatch];
 #pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (r0 < n) xs[(c0 + u) * S + r0] = v0[u];
-      if (r1 < n) xs[(c0 + u) * S + r1] = v1[u];
+      for (int u = 0; u < kRestBatch; ++u)
+        v[u] = (x + __shfl(mybase, min(c0 + u * per + cl, ncol - 1), kColBlock))[o];
+#pragma unroll
+      for (int u = 0; u < kRestBatch; ++u) {
+        const int c = c0 + u * per + cl;
+        if (cl < per && c < clast) xs[c * S + r] = v[u];
+      }
     }
   }
 }
 
 template <typename T>
-__device__ inline void stage_columns_out(const T *__restrict__ xs, int S, T *__restrict__ y,
-                                         const int *__restrict__ map, int ndf, const int *__restrict__ ind,
-                                         int n, int pos0, int nc, int cfirst = 0, int clast = kColBlock) {
+__device__ inline void stage_columns_out(const T *__restrict__ xs, int S, T *__restrict__ y, int mybase,
+                                         const int *__restrict__ ind, int n, int ncol, int cfirst, int clast) {
   const int lane = threadIdx.x & (kColBlock - 1);
-  const int mybase = pos0 + lane < nc ? map[static_cast<size_t>(pos0 + lane) * ndf] : 0;
-  const int r0 = lane, r1 = lane + kColBlock;
-  const int o0 = r0 < n ? ind[r0] : 0, o1 = r1 < n ? ind[r1] : 0;
-  const int ncol = min(kColBlock, nc - pos0);
-#pragma unroll 16
-  for (int c = cfirst; c < clast; ++c) {
-    const int base = __shfl(mybase, c, kColBlock);
-    if (c < ncol) {
-      if (r0 < n) y[static_cast<size_t>(base) + o0] = xs[c * S + r0];
-      if (r1 < n) y[static_cast<size_t>(base) + o1] = xs[c * S + r1];
+  const int full = n >= kColBlock ? kColBlock : 0, rest = n - full;
+  if (full) {
+    const long long o = ind[lane];
+#pragma unroll 1
+    for (int c0 = cfirst; c0 < clast; c0 += kStageBatch) {
+      T v[kStageBatch];
+#pragma unroll
+      for (int u = 0; u < kStageBatch; ++u) v[u] = xs[min(c0 + u, clast - 1) * S + lane];
+#pragma unroll
+      for (int u = 0; u < kStageBatch; ++u) {
+        const int base = __builtin_amdgcn_readlane(mybase, min(c0 + u, ncol - 1));
+        if (c0 + u < min(clast, ncol)) (y + base)[o] = v[u];
+      }
+    }
+  }
+  if (rest) {
+    const int per = kColBlock / rest, cl = lane / rest, r = full + (cl < per ? lane - cl * rest : 0);
+    const long long o = ind[r];
+#pragma unroll 1
+    for (int c0 = cfirst; c0 < clast; c0 += kRestBatch * per) {
+      T v[kRestBatch];
+#pragma unroll
+      for (int u = 0; u < kRestBatch; ++u) v[u] = xs[min(c0 + u * per + cl, clast - 1) * S + r];
+#pragma unroll
+      for (int u = 0; u < kRestBatch; ++u) {
+        const int c = c0 + u * per + cl, base = __shfl(mybase, min(c, ncol - 1), kColBlock);
+        if (cl < per && c < min(clast, ncol)) (y + base)[o] = v[u];
+      }
     }
   }
 }
 
-// k_cma_appinv with x and d' in LDS; c' in LDS too when CW_LDS (else in the coalesced work
-// array).  The forward sweep loads CH rows of bands at a time, so 3*CH loads are in flight per
-// lane.
-template <typename T, int CH, bool CW_LDS>
-__global__ __launch_bounds__(kColBlock) void k_cma_appinv_lds(const T *__restrict__ C, CmaP p, int nc,
+// k_cma_appinv with x and d' in LDS; c' in LDS too when CW_LDS (else in the coalesced work array).  One
+// wave a block: at C96 (864 blocks on 1024 SIMDs) nothing else hides a wave's waits, so the bands are
+// requested in two chunks of kInvChunk rows, each reloaded as soon as its rows are done, and the
+// recurrence (70 divisions one after another) runs while the next ones arrive.  C96x70 FP32: 33.0 us with
+// all bands held in registers and the fields staged a column an instruction, 22.3 us; FP64 44.9 -> 34.7 us; C24x20 FP32 22.3 -> 7.9 us.
+constexpr int kInvChunk = 10;
+constexpr int kInvBack = 24;
+
+template <typename T>
+__device__ inline void load_bands(T (&a)[kInvChunk][3], const T *__restrict__ C, int nrow, int nc, int pos, int i0) {
+#pragma unroll
+  for (int u = 0; u < kInvChunk; ++u) {  // a row past the last repeats it
+    const T *r = C + static_cast<size_t>(min(i0 + u, nrow - 1)) * 3 * nc;
+    a[u][0] = r[pos];
+    a[u][1] = (r + nc)[pos];
+    a[u][2] = (r + 2 * static_cast<size_t>(nc))[pos];
+  }
+}
+
+template <typename T, bool CW_LDS>
+__global__ __launch_bounds__(kColBlock) void k_cma_appinv_lds(const T *__restrict__ C, int nrow, int nc,
                                                               const T *__restrict__ x, T *__restrict__ y,
                                                               const int *__restrict__ map, int ndf,
                                                               const int *__restrict__ ind, T *__restrict__ cw) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T *xs = reinterpret_cast<T *>(lds_raw);
-  const int nrow = p.nrow, S = staged_stride(nrow);
+  const int S = staged_stride(nrow);
   T *cs = xs + kColBlock * S;
-  const int pos0 = blockIdx.x * kColBlock;
-  const int pos = pos0 + threadIdx.x;
-  // the first chunk of bands is requested before the staging, so the two overlap
-  T a1[CH], a2[CH], a3[CH];
-#pragma unroll
-  for (int u = 0; u < CH; ++u) {
-    const int i = 1 + u;
-    if (i > nrow || pos >= nc) continue;
-    a1[u] = C[cidx(p, nc, i, 1, pos)];
-    a2[u] = C[cidx(p, nc, i, 2, pos)];
-    a3[u] = C[cidx(p, nc, i, 3, pos)];
-  }
-  stage_columns_in<T, sizeof(T) == 4 ? 32 : kStageBatch>(xs, S, x, map, ndf, ind, nrow, pos0, nc);
+  const int pos0 = blockIdx.x * kColBlock, ncol = min(kColBlock, nc - pos0);
+  const bool mine = static_cast<int>(threadIdx.x) < ncol;
+  const int pos = min(pos0 + static_cast<int>(threadIdx.x), nc - 1);  // lanes past the last column store nothing
+  const int mybase = map[static_cast<size_t>(pos) * ndf];
+  stage_columns_in(xs, S, x, mybase, ind, nrow, ncol, 0, kColBlock);
+  T a[2][kInvChunk][3];
+  load_bands(a[0], C, nrow, nc, pos, 0);
+  load_bands(a[1], C, nrow, nc, pos, kInvChunk);
   __syncthreads();
-  if (pos < nc) {
-    T *xc = xs + threadIdx.x * S, *cc = cs + threadIdx.x * S;
-    auto cw_at = [&](int i) -> T & {
-      if constexpr (CW_LDS) return cc[i - 1];
-      else return cw[static_cast<size_t>(i - 1) * nc + pos];
-    };
-    T cprev = T(0), dprev = T(0);
-    for (int i0 = 1; i0 <= nrow; i0 += CH) {
-      if (i0 > 1) {
+  T *xc = xs + threadIdx.x * S, *cc = cs + threadIdx.x * S;
+  auto cw_at = [&](int i) -> T & {
+    if constexpr (CW_LDS) return cc[i];
+    else return cw[static_cast<size_t>(i) * nc + pos];
+  };
+  T cprev = T(0), dprev = T(0);
+  for (int i0 = 0; i0 < nrow; i0 += 2 * kInvChunk) {
 #pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int i = i0 + u;
-          if (i > nrow) continue;
-          a1[u] = C[cidx(p, nc, i, 1, pos)];
-          a2[u] = C[cidx(p, nc, i, 2, pos)];
-          a3[u] = C[cidx(p, nc, i, 3, pos)];
-        }
-      }
+    for (int h = 0; h < 2; ++h) {
+      const int ih = i0 + h * kInvChunk;
       // the chunk's right-hand sides are read from LDS before any of its results are written,
       // so the recurrence does not wait on an LDS round trip per row
-      T xv[CH];
+      T xv[kInvChunk];
 #pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int i = i0 + u;
-        if (i > nrow) continue;
-        xv[u] = xc[i - 1];
-      }
+      for (int u = 0; u < kInvChunk; ++u) xv[u] = xc[min(ih + u, nrow - 1)];
 #pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int i = i0 + u;
-        if (i > nrow) continue;
+      for (int u = 0; u < kInvChunk; ++u) {
+        const int i = ih + u;
+        if (i >= nrow) continue;
         T inv, cp, dp;
-        if (i == 1) {
-          inv = T(1) / a2[u];
-          cp = inv * a3[u];
+        if (i == 0) {
+          inv = T(1) / a[h][u][1];
+          cp = inv * a[h][u][2];
           dp = inv * xv[u];
         } else {
-          inv = T(1) / (a2[u] - a1[u] * cprev);
-          cp = i < nrow ? inv * a3[u] : T(0);
-          dp = inv * (xv[u] - a1[u] * dprev);
+          inv = T(1) / (a[h][u][1] - a[h][u][0] * cprev);
+          cp = i + 1 < nrow ? inv * a[h][u][2] : T(0);
+          dp = inv * (xv[u] - a[h][u][0] * dprev);
         }
-        cw_at(i) = cp;
-        xc[i - 1] = dp;
+        if (mine) {
+          cw_at(i) = cp;
+          xc[i] = dp;
+        }
         cprev = cp;
         dprev = dp;
       }
+      if (ih + 2 * kInvChunk < nrow) load_bands(a[h], C, nrow, nc, pos, ih + 2 * kInvChunk);
     }
-    T dnext = dprev;
-    for (int i0 = nrow - 1; i0 >= 1; i0 -= CH) {
-      T cv[CH], dv[CH];
+  }
+  T dnext = dprev;
+  for (int i0 = nrow - 2; i0 >= 0; i0 -= kInvBack) {
+    T cv[kInvBack], dv[kInvBack];
 #pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int i = i0 - u;
-        if (i < 1) continue;
-        cv[u] = cw_at(i);
-        dv[u] = xc[i - 1];
-      }
+    for (int u = 0; u < kInvBack; ++u) {
+      const int i = max(i0 - u, 0);
+      cv[u] = cw_at(i);
+      dv[u] = xc[i];
+    }
 #pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int i = i0 - u;
-        if (i < 1) continue;
-        const T d = dv[u] - cv[u] * dnext;
-        xc[i - 1] = d;
-        dnext = d;
-      }
+    for (int u = 0; u < kInvBack; ++u) {
+      const int i = i0 - u;
+      if (i < 0) continue;
+      const T d = dv[u] - cv[u] * dnext;
+      if (mine) xc[i] = d;
+      dnext = d;
     }
   }
   __syncthreads();
-  stage_columns_out(xs, S, y, map, ndf, ind, nrow, pos0, nc);
+  stage_columns_out(xs, S, y, mybase, ind, nrow, ncol, 0, kColBlock);
 }
 
 // k_cma_apply<T, BW> for 64 columns per block of kApplyWaves wavefronts: the waves stage x
@@ -422,15 +455,18 @@ void k_cma_apply_lds(
   const int Sx = staged_stride(p.ncol), Sy = staged_stride(p.nrow);
   T *ys = xs + kColBlock * Sx;
   const int pos0 = blockIdx.x * kColBlock;
-  const int w = threadIdx.x / kColBlock, lane = threadIdx.x & (kColBlock - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kColBlock), lane = threadIdx.x & (kColBlock - 1);
+  const int ncol = min(kColBlock, nc - pos0);
   constexpr int kCw = kColBlock / kApplyWaves;
   const int pos = pos0 + lane;
   const int q = (p.nrow + kApplyWaves - 1) / kApplyWaves;
   const int ifirst = 1 + w * q, ilast = min(p.nrow, (w + 1) * q);
   T a[kApplyChunk][BW];
   if (pos < nc) load_band_chunk<T, BW>(a, C, p, nc, pos, ifirst, ilast);
-  stage_columns_in(xs, Sx, x, map_from, ndf_from, ind_from, p.ncol, pos0, nc, w * kCw, (w + 1) * kCw);
-  if (accumulate) stage_columns_in(ys, Sy, y, map_to, ndf_to, ind_to, p.nrow, pos0, nc, w * kCw, (w + 1) * kCw);
+  const int bf = map_from[static_cast<size_t>(min(pos, nc - 1)) * ndf_from];
+  const int bt = map_to[static_cast<size_t>(min(pos, nc - 1)) * ndf_to];
+  stage_columns_in(xs, Sx, x, bf, ind_from, p.ncol, ncol, w * kCw, (w + 1) * kCw);
+  if (accumulate) stage_columns_in(ys, Sy, y, bt, ind_to, p.nrow, ncol, w * kCw, (w + 1) * kCw);
   __syncthreads();
   if (pos < nc) {
     const T *xc = xs + lane * Sx;
@@ -453,7 +489,7 @@ void k_cma_apply_lds(
     }
   }
   __syncthreads();
-  stage_columns_out(ys, Sy, y, map_to, ndf_to, ind_to, p.nrow, pos0, nc, w * kCw, (w + 1) * kCw);
+  stage_columns_out(ys, Sy, y, bt, ind_to, p.nrow, ncol, w * kCw, (w + 1) * kCw);
 }
 
 // columnwise_op_mul_kernel_code (sci_columnwise_op_mul_kernel_mod.F90:128-160): C += A B.
@@ -764,19 +800,19 @@ int launch_cma_appinv(const lfric_cma *A, const void *x, void *y) {
     const int blocks = (A->ncols + kColBlock - 1) / kColBlock;
     const bool cw_lds = 2 * lds1 <= 64 * 1024;  // c' beside x while four blocks still fit a CU
     const size_t lds = cw_lds ? 2 * lds1 : lds1;
-#define APPINV_LDS(T, CH)                                                                                       \
-  if (cw_lds)                                                                                                   \
-    hipLaunchKernelGGL((k_cma_appinv_lds<T, CH, true>), dim3(blocks), dim3(kColBlock), lds, cur_stream(),       \
-                       static_cast<const T *>(A->d), p, A->ncols, static_cast<const T *>(x), static_cast<T *>(y), \
-                       f.d_map, f.ndf, A->d_ind_to, static_cast<T *>(A->work));                                 \
-  else                                                                                                          \
-    hipLaunchKernelGGL((k_cma_appinv_lds<T, CH, false>), dim3(blocks), dim3(kColBlock), lds, cur_stream(),      \
-                       static_cast<const T *>(A->d), p, A->ncols, static_cast<const T *>(x), static_cast<T *>(y), \
-                       f.d_map, f.ndf, A->d_ind_to, static_cast<T *>(A->work));
+#define APPINV_LDS(T)                                                                                            \
+  if (cw_lds)                                                                                                    \
+    hipLaunchKernelGGL((k_cma_appinv_lds<T, true>), dim3(blocks), dim3(kColBlock), lds, cur_stream(),            \
+                       static_cast<const T *>(A->d), A->nrow, A->ncols, static_cast<const T *>(x),               \
+                       static_cast<T *>(y), f.d_map, f.ndf, A->d_ind_to, static_cast<T *>(A->work));             \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_cma_appinv_lds<T, false>), dim3(blocks), dim3(kColBlock), lds, cur_stream(),           \
+                       static_cast<const T *>(A->d), A->nrow, A->ncols, static_cast<const T *>(x),               \
+                       static_cast<T *>(y), f.d_map, f.ndf, A->d_ind_to, static_cast<T *>(A->work));
     if (A->precision == LFRIC_R64) {
-      APPINV_LDS(double, 36)
+      APPINV_LDS(double)
     } else {
-      APPINV_LDS(float, 72)
+      APPINV_LDS(float)
     }
 #undef APPINV_LDS
     return finish("columnwise inverse");

@@ -141,6 +141,14 @@ def test_cma_tall_columns_bitwise_equal_oracle(hip, orc, P, nl):
     np.testing.assert_array_equal(y.export_raw(), orc.cma_appinv(pc, ref, x, dm3, i3, r32=r32))
 
 
+@pytest.mark.parametrize("P", ["R32", "R64"])
+@pytest.mark.parametrize("nl", [1, 2, 21, 40, 63, 64, 65, 70, 127])
+def test_cma_staged_heights_bitwise_equal_oracle(hip, orc, P, nl):
+    """The same checks at the heights where the staging changes: several columns an instruction (below
+    64 rows), none left over (64), one and 63 rows left over (65, 127), one to several chunks of bands."""
+    test_cma_tall_columns_bitwise_equal_oracle(hip, orc, P, nl)
+
+
 def test_cma_diag_hmht_bitwise_equals_oracle(hip, orc):
     """asm_diag_hmht from a W3 <- W2h LMA operator and a W2h mass (the side faces of the box's W2
     dofmap, shared between neighbouring cells)."""
