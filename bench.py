@@ -64,8 +64,10 @@ def solve_roofline(fs, mres, pres, t_mixed, t_fp64, packed=False):
     divided by the solve time.  Iteration: the apply with p.(A p) (matrix, x, y, dofmap once
     each; the matrix counted as the triangles it reads when the apply is the symmetric-packed
     one), the update (reads x, p, r, A p, diag; writes x, r, z: 8 vector passes) and aypx
-    (reads z, p; writes p: 3), i.e. 11 vector passes of undf entries beyond the apply."""
-    passes = 11
+    (reads z, p; writes p: 3), i.e. 11 vector passes of undf entries beyond the apply.  Over the
+    symmetric copy A p is not stored: the gather reads r, diag and writes r, z, the step reads x, p,
+    z and writes x, p, and the apply's y is not written, 8 passes beyond the apply."""
+    passes = 8 if packed else 11
     ab = (lambda s: sym_bytes(fs, s, s)) if packed else (lambda s: apply_bytes(fs, 8, s, s))
     it32 = ab(4) + passes * fs.undf * 4
     it64 = ab(8) + passes * fs.undf * 8
@@ -628,10 +630,10 @@ def helmholtz_record(L, reps=3):
     res64 = plain_runs[-1][1]
     x32, y32 = L.FieldVector(w3, L.R32).fill_uniform(1, 3), L.FieldVector(w3, L.R32)
     t_apply = time_applies(L, H32, x32, y32, 20, "apply")
-    # one H apply: D^T (6 entries per cell-layer) and D read once each, M3 once; x read twice, the
-    # W2 intermediate written and read, y written
+    # one H apply (one kernel): D's 6 entries of a cell-layer and its 4 side neighbours' and M3 from the
+    # composite's copy, diag(M2) and x read once, y written
     nc3 = w3.ncell_3d
-    apply_bytes = nc3 * (6 + 6 + 1) * 4 + w3.undf * 3 * 4 + w2.undf * 2 * 4
+    apply_bytes = nc3 * (6 + 4 + 1) * 4 + w3.undf * 2 * 4 + w2.undf * 4
     return {
         "workload": "C48x50 W2/W3 Helmholtz-like H = M3 + 0.5 D diag(M2)^-1 D^T on W3 (691,200 dofs), GMRES(30) "
                     "to 1e-8: FP32 applies, BF16 column block-Jacobi, FP64 refinement and Givens",
