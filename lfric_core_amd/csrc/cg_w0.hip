@@ -42,7 +42,8 @@ __device__ inline void record(SolverState *st, const Test &t, int it) {
 // neighbours still read the old one.  With it = 0 p is z.
 //   Bound: latency.  Forming p here doubles the loads of x but leaves two launches of the three (gather, update,
 // aypx: 6.6 + 5.7 + 6.5 us at C12x20, FP64); a point's element rows are requested before the partials are added.
-template <typename T>
+// AHEAD: so are z and the old p, which takes 364 registers in FP64 (one wave on a SIMD).
+template <typename T, bool AHEAD>
 __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A, size_t gs,
                                                         const W0Col *__restrict__ tab, const T *__restrict__ z,
                                                         const T *__restrict__ pold, T *__restrict__ pnew,
@@ -75,6 +76,22 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A,
       bot[k][c] = k < cnt && has_m ? *reinterpret_cast<const VecT *>(rb + static_cast<size_t>(c) * 64 * V) : VecT{};
     }
   }
+  T zl[AHEAD ? 4 : 1][3][4], pl[AHEAD ? 4 : 1][3][4];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int c4[4] = {xc[k].x, xc[k].y, xc[k].z, xc[k].w};
+#pragma unroll
+      for (int l = 0; l < 3; ++l)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // dof 0 where there is no such point
+          const int d = k < cnt && (l > 0 || has_p) && (l < 2 || has_m) ? c4[j] + m + l - 1 : 0;
+          zl[k][l][j] = z[d];
+          pl[k][l][j] = pold[d];
+        }
+    }
+  }
   __builtin_amdgcn_sched_barrier(0);
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   T b = T(0);
@@ -99,9 +116,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A,
     T xl[3][4];  // p of the cell's 4 columns at levels m-1, m, m+1
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      xl[0][j] = has_p ? pf(c4[j] + m - 1) : T(0);
-      xl[1][j] = pf(c4[j] + m);
-      xl[2][j] = has_m ? pf(c4[j] + m + 1) : T(0);
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int l = 0; l < 3; ++l) xl[l][j] = fma(b, pl[k][l][j], zl[k][l][j]);
+      } else {
+        xl[0][j] = has_p ? pf(c4[j] + m - 1) : T(0);
+        xl[1][j] = pf(c4[j] + m);
+        xl[2][j] = has_m ? pf(c4[j] + m + 1) : T(0);
+      }
     }
     if (has_p) {
 #pragma unroll
@@ -172,6 +194,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_test(SolverState *st, int it, 
   if (threadIdx.x == 0) record(st, t, it);
 }
 
+constexpr int kAheadBlocks = 256;  // compute units
+
 template <typename T>
 int iteration_t(const lfric_op *op, void *const (&v)[6], const T *diag, SolverState *st, int it) {
   const FunctionSpace &f = *op->to;
@@ -179,7 +203,11 @@ int iteration_t(const lfric_op *op, void *const (&v)[6], const T *diag, SolverSt
   T *x = static_cast<T *>(v[0]), *r = static_cast<T *>(v[1]), *z = static_cast<T *>(v[2]), *q = static_cast<T *>(v[3]);
   T *pold = static_cast<T *>(v[4 + (it & 1)]), *pnew = static_cast<T *>(v[4 + ((it + 1) & 1)]);
   double *part = ctx().d_partials, *pq = part + 2 * kCgW0Blocks;
-  hipLaunchKernelGGL(k_cg_w0_apply<T>, dim3(nb), dim3(kBlock), 0, cur_stream(), static_cast<const T *>(op->d), op->gs,
+  // loads ahead while all blocks are resident at once (a wave on a SIMD in FP64, two in FP32).  Solves without -> with,
+  // FP64: C12x20 (72 blocks) 283 -> 257 us, C20x25 (244) 321 -> 288, C24x30 (419) 423 -> 438; FP32: C12x20 167 -> 149,
+  // C24x36 (500) 216 -> 191
+  auto apply = nb <= (sizeof(T) == 4 ? 2 : 1) * kAheadBlocks ? k_cg_w0_apply<T, true> : k_cg_w0_apply<T, false>;
+  hipLaunchKernelGGL(apply, dim3(nb), dim3(kBlock), 0, cur_stream(), static_cast<const T *>(op->d), op->gs,
                      static_cast<const W0Col *>(f.d_w0tab), z, it > 0 ? pold : z, pnew, q, f.w0tab_cols, f.nlayers, st,
                      it, part, nb, pq);
   hipLaunchKernelGGL(k_cg_w0_update<T>, dim3(nb), dim3(kBlock), 0, cur_stream(), x, r, z, pnew, q, diag, n, st, it, pq,
