@@ -64,10 +64,8 @@ def solve_roofline(fs, mres, pres, t_mixed, t_fp64, packed=False):
     divided by the solve time.  Iteration: the apply with p.(A p) (matrix, x, y, dofmap once
     each; the matrix counted as the triangles it reads when the apply is the symmetric-packed
     one), the update (reads x, p, r, A p, diag; writes x, r, z: 8 vector passes) and aypx
-    (reads z, p; writes p: 3), i.e. 11 vector passes of undf entries beyond the apply.  Over the
-    symmetric copy A p is not stored: the gather reads r, diag and writes r, z, the step reads x, p,
-    z and writes x, p, and the apply's y is not written, 8 passes beyond the apply."""
-    passes = 8 if packed else 11
+    (reads z, p; writes p: 3), i.e. 11 vector passes of undf entries beyond the apply."""
+    passes = 11
     ab = (lambda s: sym_bytes(fs, s, s)) if packed else (lambda s: apply_bytes(fs, 8, s, s))
     it32 = ab(4) + passes * fs.undf * 4
     it64 = ab(8) + passes * fs.undf * 8

@@ -8,7 +8,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "liblfric_hip.so"
 SOURCES = ["api.hip", "kernels.hip", "krylov.hip", "solvers.hip", "batch.hip", "cma.hip", "order1_apply.hip",
-           "w0_apply.hip", "w2_apply.hip", "mrhs_apply.hip", "cg_sym.hip", "cg_w0.hip",
+           "w0_apply.hip", "w2_apply.hip", "mrhs_apply.hip", "cg_w0.hip",
            "mesh_gen.cpp", "ugrid.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

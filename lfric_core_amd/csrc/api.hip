@@ -338,8 +338,7 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
   const double *pzp = fused ? pz_partials : c.d_partials;
   const int npz = fused ? pz_blocks : kRedBlocks;
   const bool fold = npz <= kFoldMaxPartials;
-  const bool sym = fused && cg_sym_usable(a.A);
-  if (fused && !sym && cg_w0_usable(a.A)) {
+  if (fused && cg_w0_usable(a.A)) {
     void *v[6] = {a.x, r, z, nullptr, p, nullptr};
     if (scratch_base) {
       cg_scratch_layout(vb, pz_blocks, soff);
@@ -364,10 +363,6 @@ static int cg_device(const CgArgs &a, SolverState &out, unsigned char *scratch_b
   for (int ch = 0; ch < max_chunks; ++ch) {
     for (int i = 0; i < every; ++i, ++it) {
       const int par = static_cast<int>(it & 1);
-      if (sym) {
-        if (int rc = launch_cg_sym_iteration(a.A, a.x, r, z, p, a.diag, g_state, it)) return rc;
-        continue;
-      }
       if (fused) {
         if (int rc = launch_lma_apply_gather_dot(a.A, p, z, pz_partials, &g_state->done)) return rc;
       } else {
@@ -426,7 +421,7 @@ int lfric_init(int device) {
   LF_HIP(hipEventCreate(&c.t0));
   LF_HIP(hipEventCreate(&c.t1));
   c.device = device;
-  c.partials_cap = static_cast<size_t>(kRedBlocks) * 4 + kSymUnitPartials;
+  c.partials_cap = static_cast<size_t>(kRedBlocks) * 4;
   if (int rc = dmalloc(reinterpret_cast<void **>(&c.d_partials), sizeof(double) * c.partials_cap)) return rc;
   if (int rc = dmalloc(reinterpret_cast<void **>(&c.d_counter), sizeof(unsigned int) * 16)) return rc;
   LF_HIP(hipMemset(c.d_counter, 0, sizeof(unsigned int) * 16));

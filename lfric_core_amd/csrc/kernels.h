@@ -18,7 +18,7 @@ struct SolverState {
   double red0, red1;  // last reduction results
   int iter, max_iter, done, status, monitor, converged;
   unsigned int counter;
-  int stop;  // the iteration over the symmetric-packed copy: phase + 1 of the kernel that ended the solve
+  int pad;
 };
 
 constexpr int kRedBlocks = 2048;  // fixed grid of the reduction kernels (deterministic sums)
@@ -140,14 +140,6 @@ int launch_cg_update(int prec, void *x, void *r, void *z, const void *p, const v
 // convergence test, beta and p = z + beta p from the update's partials
 int launch_cg_aypx(int prec, void *p, const void *z, long long n, SolverState *st, int par);
 int launch_cg_finish_pz(const double *partials, int nblocks, SolverState *st, int par);
-// one iteration over the symmetric-packed copy (one unit per thread): three kernels, on the same state,
-// scalars and operation order; it counts the iterations enqueued.  Usable while its first kernel's partials
-// fit the context's buffer (beyond its first 4 * kRedBlocks); cg_sym.hip
-constexpr int kSymUnitPartials = 32768;
-int cg_sym_partials(const lfric_op *op);
-bool cg_sym_usable(const lfric_op *op);
-int launch_cg_sym_iteration(const lfric_op *op, void *x, void *r, void *z, void *p, const void *diag, SolverState *st,
-                            long long it);
 // one iteration over the element layout of a lowest-order W0 operator in two kernels, for small problems: v =
 // x, r, z, q, and the two buffers of p.  The first kernel of an iteration tests the one before, so the host's reads
 // follow launch_cg_w0_test; cg_w0.hip

@@ -35,7 +35,6 @@
 #include "role_kind.h"
 #include "rng.h"
 #include "sym27_apply.h"
-#include "sym_apply.h"
 
 namespace lfric {
 
@@ -784,6 +783,8 @@ __global__ __launch_bounds__(kBlock) void k_lma_gather_rows_w0(const T *__restri
 // triangles: slot s is layer seg*S - 1 + s (slot 0 repeats the previous segment's last one).
 // Entry k of slot s of thread t sits at (t/64)*gss + ((s*NCH + k/V)*64 + t%64)*V + k%V, NCH =
 // 36/V chunks, so each wavefront load is one contiguous 1 KiB block.
+__host__ __device__ constexpr int tri_index(int i, int j) { return i * 8 - i * (i - 1) / 2 + (j - i); }
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_build_sym(const T *__restrict__ A, size_t gs, const int *__restrict__ ebase,
                                                       T *__restrict__ sym, size_t gss, int ncells, int nl, int S,
@@ -947,8 +948,15 @@ __global__ __launch_bounds__(kBlock) void k_sym_units_s(const T *__restrict__ sy
   }
 }
 
-// One unit per thread (the default copy): sym_apply.h.  slotpos[k]: the colour-major position of the cell of
-// slot k.
+// One unit per thread (the default copy).  Cells take slots in cell-id order, so that the
+// threads of a window of blocks work on neighbouring cells and share their x entries in one
+// L2: unit t = k*(nl+1) + m is (k-th cell, level m), the cell at colour-major position
+// slotpos[k].  Slot t of the copy holds the triangle of that cell's layer-m element (m < nl; the
+// slot of m = nl is empty), entry q at (t/64)*gss + ((q/V)*64 + t%64)*V + q%V.  A unit's thread
+// forms the bottom rows' chains c_i of its element (x at levels m, m+1) and the top rows' chains
+// of the same element, which belong to unit m+1: the next lane takes them with one shuffle.
+// Every chain is the colour kernel's (same entries, same x, same order); the unit's 4 outputs
+// go to z[(k*4 + i)*(nl+1) + m].
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_build_sym1(const T *__restrict__ A, size_t gs, const int *__restrict__ ebase,
                                                        const int *__restrict__ slotpos, T *__restrict__ sym, size_t gss,
@@ -979,19 +987,71 @@ __global__ __launch_bounds__(kBlock) void k_build_sym1(const T *__restrict__ A, 
   if (mismatch) *asym = 1;
 }
 
-// phase 1: the unit's 4 outputs go to z[(k*4 + i)*(nl+1) + m]
+// cellcol[k]: the 0-based base dofs of the k-th cell's 4 bottom vertex columns.  A wavefront
+// takes 63 new units and repeats, in lane 0, the previous wavefront's last unit (whose outputs
+// it does not write), so that every unit's lower neighbour is the previous lane; s1_threads
+// gives the launch's thread count.
+inline long long s1_threads(long long units) { return (units + 62) / 63 * 64; }
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_sym_units1(const T *__restrict__ sym, size_t gss, const T *__restrict__ x,
                                                        const int4 *__restrict__ cellcol, T *__restrict__ z, int ncells,
                                                        int nl, const int *skip, int xwin) {
   if (skip && *skip) return;
+  constexpr int V = chunk_entries<T>(), NCH = 36 / V;
+  typedef T VecT __attribute__((ext_vector_type(V)));
+  const int H = nl + 1;
   const long long g = static_cast<long long>(xcd_block(blockIdx.x, gridDim.x, xwin)) * kBlock + threadIdx.x;
-  int k, m;
-  T x0[4], out[4];
-  if (!sym_unit<T>(sym, gss, x, cellcol, ncells, nl, g, k, m, x0, out)) return;
-  T *zp = z + static_cast<size_t>(k) * 4 * (nl + 1);
+  const int lane = threadIdx.x & 63;
+  const long long t = (g >> 6) * 63 + lane - 1;
+  const bool valid = t >= 0 && t < static_cast<long long>(ncells) * H;
+  const int k = valid ? static_cast<int>(t / H) : 0;
+  const int m = valid ? static_cast<int>(t - static_cast<long long>(k) * H) : 0;
+  const bool has_m = valid && m < nl, has_p = valid && m > 0;
+  const long long tc = valid ? t : 0;
+  const T *St = sym + static_cast<size_t>(tc >> 6) * gss + static_cast<size_t>(tc & 63) * V;
+  VecT tri[NCH];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) zp[static_cast<size_t>(i) * (nl + 1) + m] = out[i];
+  for (int c = 0; c < NCH; ++c)
+    tri[c] = has_m ? __builtin_nontemporal_load(reinterpret_cast<const VecT *>(St + static_cast<size_t>(c) * 64 * V))
+                   : VecT{};
+  int b[4] = {0, 0, 0, 0};
+  if (valid) {
+    const int4 bb = cellcol[k];
+    b[0] = bb.x;
+    b[1] = bb.y;
+    b[2] = bb.z;
+    b[3] = bb.w;
+  }
+  T x0[4], x1[4];  // x at levels m and m+1
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    x0[j] = valid ? x[b[j] + m] : T(0);
+    x1[j] = has_m ? x[b[j] + m + 1] : T(0);
+  }
+  auto at = [&](int q) { return tri[q / V][q % V]; };
+  T c[4], cn[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    T s = T(0), sn = T(0);
+    if (has_m) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s = fma(at(j >= i ? tri_index(i, j) : tri_index(j, i)), j < 4 ? x0[j] : x1[j - 4], s);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        sn = fma(at(j >= i + 4 ? tri_index(i + 4, j) : tri_index(j, i + 4)), j < 4 ? x0[j] : x1[j - 4], sn);
+    }
+    c[i] = s;
+    cn[i] = sn;
+  }
+  // the top rows of the layer-(m-1) element: the previous lane's unit (m-1 of the same cell)
+  T cp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cp[i] = __shfl_up(cn[i], 1, 64);
+  if (!valid || lane == 0) return;
+  T *zp = z + static_cast<size_t>(k) * 4 * H;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) zp[static_cast<size_t>(i) * H + m] = c[i] + (has_p ? cp[i] : T(0));
 }
 
 // phase 2: y at (column, level) = the units' outputs of the column's cells in colour order, the

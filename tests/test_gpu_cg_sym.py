@@ -1,9 +1,16 @@
-"""Conjugate gradients over the symmetric-packed copy, whose iteration forms p.(A p) from the units and
-updates the residual where it gathers A p, against the same solve over the element layout: the operators are
-the same and only the order of a sum changes, so the iteration counts agree within one and the solutions to
-what a residual of r_tol leaves (condition of B B^T + 0.1 I elements below 100: 100 r_tol).  Sizes with one
-block and several, partial blocks and wavefronts; and the ends of a solve: no iteration (b = 0 and an exact
-initial guess), the iteration limit, monitoring off."""
+"""Conjugate gradients over the symmetric-packed copy.
+
+* Against the same solve over the element layout: the operators are the same and only the order of a sum
+  changes, so the iteration counts agree within one and the solutions to what a residual of r_tol leaves
+  (condition of B B^T + 0.1 I elements below 100: 100 r_tol).  Sizes with one block and several, partial blocks
+  and wavefronts; and the ends of a solve: no iteration (b = 0 and an exact initial guess), the iteration limit,
+  monitoring off.
+* Against the iteration written out in the public vector operations, bit for bit, over systems whose columns
+  are scaled by 10^U(-2, 2): hundreds of FP32 iterations carry one rounding of alpha to another stopping
+  point, so the products have to be those of the vectors themselves (p . (A p) of the gathered A p).  Up to
+  2048 blocks of 256 dofs a dot's partial sums are the apply's.
+* The scaled mixed-precision solve against its refinement written out the same way, and its residual in
+  the oracle's assembled matrix."""
 import numpy as np
 import pytest
 
@@ -59,3 +66,86 @@ def test_ends_of_a_solve(hip):
     x.set_scalar(0.0)
     with pytest.raises(hip.LfricError):
         hip.ConjugateGradient(op, prec, 1e-10, 0.0, 50).apply(x, bad)
+
+
+def _scaled_system(hip, n, nl, copy, prec):
+    fs = hip.FunctionSpace.cubedsphere(n, nl)
+    op64 = hip.LmaOperator(fs).generate_spd(n + nl, scaled=True)
+    ops = [op64, op64.convert(hip.R32)] if prec == "mixed" else [op64 if prec == "R64" else op64.convert(hip.R32)]
+    for op in ops:
+        if copy == "rows":
+            op.prepare_rows()
+        elif copy == "symmetric":
+            op.prepare_symmetric()
+    return (fs, *ops)
+
+
+def _cg_by_vector_operations(hip, op, diag, b, iterations):
+    """x after each iteration from x = 0 (cg_solve without a convergence test)."""
+    A = hip.LinearOperator.from_lma(op)
+    x, r, z, p, q = (b.duplicate() for _ in range(5))
+    x.set_scalar(0.0)
+    r.copy(b)
+    z.divide(r, diag)
+    p.copy(z)
+    rz = r.dot(z)
+    for _ in range(iterations):
+        A.apply(p, q)
+        alpha = rz / p.dot(q)
+        x.axpy(alpha, p)
+        r.axpy(-alpha, q)
+        z.divide(r, diag)
+        rz, old = r.dot(z), rz
+        p.aypx(rz / old, z)
+    return x
+
+
+@pytest.mark.parametrize("prec", ["R64", "R32"])
+@pytest.mark.parametrize("copy", ["none", "rows", "symmetric"])
+@pytest.mark.parametrize("n,nl", [(4, 62), (12, 20), (32, 60)])
+def test_scaled_cg_equals_the_vector_operations(hip, n, nl, copy, prec):
+    P = getattr(hip, prec)
+    fs, op = _scaled_system(hip, n, nl, copy, prec)
+    diag = op.mm_diagonal(hip.FieldVector(fs, P))
+    b = hip.FieldVector(fs, P).fill_uniform(n, 3)
+    for iters in (7, 60):
+        x = hip.FieldVector(fs, P)
+        x.set_scalar(0.0)
+        res = hip.ConjugateGradient(op, hip.DiagonalPreconditioner(diag), 1e-30, 0.0, iters, monitor_convergence=False,
+                                    check_every=16).apply(x, b)
+        assert res.iterations == iters
+        np.testing.assert_array_equal(x.export_raw(), _cg_by_vector_operations(hip, op, diag, b, iters).export_raw())
+
+
+@pytest.mark.parametrize("copy", ["none", "rows", "symmetric"])
+def test_scaled_mixed_precision_solve(hip, orc, copy):
+    fs, op, op32 = _scaled_system(hip, 8, 12, copy, "mixed")
+    prec = hip.DiagonalPreconditioner.from_operator(op32)
+    b, x = hip.FieldVector(fs).fill_uniform(1, 3), hip.FieldVector(fs)
+    A, want = hip.LinearOperator.from_lma(op), np.zeros(fs.undf)
+    for outer in range(2):
+        # r = b - A x, its inner solve to the remaining reduction, and x + ||r|| d
+        xw, r = hip.FieldVector(fs).import_field(want), hip.FieldVector(fs)
+        A.apply(xw, r)
+        r.import_field(b.export_field() - r.export_field())
+        nr = r.norm()
+        nr0 = nr if outer == 0 else nr0
+        b32, d32 = hip.FieldVector(fs, hip.R32), hip.FieldVector(fs, hip.R32)
+        b32.import_raw((r.export_field() * (1.0 / nr)).astype(np.float32))
+        d32.set_scalar(0.0)
+        hip.ConjugateGradient(op32, prec, max(1e-4, 0.5 * 1e-8 * nr0 / nr), 0.0, 2000).apply(d32, b32)
+        want = want + nr * d32.export_raw().astype(np.float64)
+        x.set_scalar(0.0)
+        res = hip.MixedPrecisionCG(op, op32, prec, 1e-8, 0.0, 2000, max_outer=outer + 1).apply(x, b)
+        assert res.outer_iterations == outer + 1
+        got = x.export_field()
+        # the device adds nr d to x with or without rounding the product first
+        assert np.all(np.abs(got - want) <= np.finfo(np.float64).eps * (np.abs(got) + np.abs(want)))
+        want = got
+    x.set_scalar(0.0)
+    res = hip.MixedPrecisionCG(op, op32, prec, 1e-8, 0.0, 2000).apply(x, b)
+    assert res.status == 0
+    m = orc.Mesh(8, 12)
+    S = orc.assembled_csr(m, orc.gen_spd(m.ndf, m.ncell_3d, 20, scaled=True))
+    bb = b.export_field()
+    assert np.linalg.norm(bb - S @ x.export_field()) <= 1e-8 * np.linalg.norm(bb)
