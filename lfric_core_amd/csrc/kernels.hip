@@ -2371,14 +2371,11 @@ int launch_sym27_mrhs(const lfric_op *op, const void *x, void *y, int nrhs) {
 }
 
 template <typename T, int N2, class R>
-static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, GatherExtra ex) {
+static int launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, GatherExtra ex) {
   const FunctionSpace &to = *op->to, &from = *op->from;
   const int grid = gather_blocks(op);
   if constexpr (N2 == 27 && std::is_same<R, RolesW0K1>::value) {
-    if (sym27_ready(op)) {
-      (void)launch_sym27<T, 1>(op, x, y, ex.partials, ex.skip);
-      return;
-    }
+    if (sym27_ready(op)) return launch_sym27<T, 1>(op, x, y, ex.partials, ex.skip);
   }
   if constexpr (N2 == 8 && std::is_same<R, RolesW0K0>::value) {
     if (op->sym) {  // symmetric-packed copy (launch_build_sym): two phases
@@ -2407,7 +2404,7 @@ static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gathe
                grid_for(static_cast<long long>(to.gather_ncols) * (to.nlayers + 1), kBlock * kSymPoints),
                static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent,
                op->d_symzu, to.gather_ncols, to.nlayers, ex.skip, op->xwin);
-      return;
+      return LFRIC_OK;
     }
     if (op->rows) {  // built only for square lowest-order W0 operators (launch_build_rows)
       const T *rw = static_cast<const T *>(op->rows);
@@ -2417,18 +2414,12 @@ static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gathe
       else
         LAUNCH((k_lma_gather_rows_w0<T, false>), grid, rw, op->gsr, x, y, from.d_map, to.d_gcol, to.d_goff,
                to.d_gent, to.gather_ncols, to.nlayers, ex.partials, ex.skip, op->xwin);
-      return;
+      return LFRIC_OK;
     }
-    if (to.d_w0tab && op->to == op->from) {
-      (void)launch_w0_gather(op, x, y, false, ex.partials, ex.skip);
-      return;
-    }
+    if (to.d_w0tab && op->to == op->from) return launch_w0_gather(op, x, y, false, ex.partials, ex.skip);
   }
   if constexpr (N2 == 6 && std::is_same<R, RolesW2K0>::value) {
-    if (to.d_w2col && op->to == op->from) {
-      (void)launch_w2_gather(op, x, y, false, ex.partials, ex.skip, 0);
-      return;
-    }
+    if (to.d_w2col && op->to == op->from) return launch_w2_gather(op, x, y, false, ex.partials, ex.skip, 0);
   }
   if (ex.partials)
     LAUNCH((k_lma_gather<T, N2, R, true>), grid, static_cast<const T *>(op->d), op->gs, to.d_ebase, x, y, from.d_map,
@@ -2436,16 +2427,17 @@ static void launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gathe
   else
     LAUNCH((k_lma_gather<T, N2, R, false>), grid, static_cast<const T *>(op->d), op->gs, to.d_ebase, x, y,
            from.d_map, to.d_gcol, to.d_goff, to.d_gent, to.gather_ncols, to.nlayers, roles, ex.partials, ex.skip, op->xwin);
+  return LFRIC_OK;
 }
 
 template <typename T, int N2>
-static void launch_gather_n(RoleKind rk, const lfric_op *op, const T *x, T *y, GatherExtra ex) {
+static int launch_gather_n(RoleKind rk, const lfric_op *op, const T *x, T *y, GatherExtra ex) {
   switch (rk) {
-    case RoleKind::W0K0: launch_gather_r<T, N2>(op, x, y, RolesW0K0{}, ex); break;
-    case RoleKind::W0K1: launch_gather_r<T, N2>(op, x, y, RolesW0K1{}, ex); break;
-    case RoleKind::W2K0: launch_gather_r<T, N2>(op, x, y, RolesW2K0{}, ex); break;
-    case RoleKind::None: launch_gather_r<T, N2>(op, x, y, RolesNone{}, ex); break;
-    default: launch_gather_r<T, N2>(op, x, y, RolesRuntime{roles_of(*op->to)}, ex);
+    case RoleKind::W0K0: return launch_gather_r<T, N2>(op, x, y, RolesW0K0{}, ex);
+    case RoleKind::W0K1: return launch_gather_r<T, N2>(op, x, y, RolesW0K1{}, ex);
+    case RoleKind::W2K0: return launch_gather_r<T, N2>(op, x, y, RolesW2K0{}, ex);
+    case RoleKind::None: return launch_gather_r<T, N2>(op, x, y, RolesNone{}, ex);
+    default: return launch_gather_r<T, N2>(op, x, y, RolesRuntime{roles_of(*op->to)}, ex);
   }
 }
 
@@ -2453,14 +2445,16 @@ template <typename T>
 static int gather_t(const lfric_op *op, const T *x, T *y, GatherExtra ex) {
   if (int rc = build_gather(*op->to)) return rc;
   const RoleKind rk = role_kind(*op->to);
+  int rc = LFRIC_OK;  // a launcher that checks its own launch has taken the error from hipGetLastError
   switch (op->from->ndf) {
-    case 1: launch_gather_n<T, 1>(rk, op, x, y, ex); break;
-    case 2: launch_gather_n<T, 2>(rk, op, x, y, ex); break;
-    case 6: launch_gather_n<T, 6>(rk, op, x, y, ex); break;
-    case 8: launch_gather_n<T, 8>(rk, op, x, y, ex); break;
-    case 27: launch_gather_n<T, 27>(rk, op, x, y, ex); break;
+    case 1: rc = launch_gather_n<T, 1>(rk, op, x, y, ex); break;
+    case 2: rc = launch_gather_n<T, 2>(rk, op, x, y, ex); break;
+    case 6: rc = launch_gather_n<T, 6>(rk, op, x, y, ex); break;
+    case 8: rc = launch_gather_n<T, 8>(rk, op, x, y, ex); break;
+    case 27: rc = launch_gather_n<T, 27>(rk, op, x, y, ex); break;
     default: return fail(LFRIC_E_UNSUPPORTED, "lma_apply_gather: unsupported ndf_from");
   }
+  if (rc) return rc;
   CHECK_LAUNCH();
   return LFRIC_OK;
 }
