@@ -25,6 +25,16 @@ __device__ inline Test test_of(const SolverState *st, const double *__restrict__
   t.conv = !t.nan && st->monitor && (t.rn / st->r_nrm0 <= st->r_tol || t.rn <= st->a_tol);
   return t;
 }
+// Whether the solve has ended before this kernel.  The update does not set `done` on a NaN or zero p.q but
+// leaves that to the kernel after it, here: set there, `done` would be read by the later waves of blocks whose
+// earlier waves started without it, and such a block would add an incomplete p.q and step x with it.
+// (record sets `done` while blocks of the apply start; a block it divides writes p and q alone, which a solve that
+// has ended does not read.)
+__device__ inline bool ended(SolverState *st, bool lead) {
+  if (!st->done && !st->status) return false;
+  if (lead) st->done = 1;
+  return true;
+}
 // one thread: the state after `it` iterations
 __device__ inline void record(SolverState *st, const Test &t, int it) {
   st->iter = it;
@@ -50,7 +60,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A,
                                                         T *__restrict__ q, int ncols, int nl, SolverState *st, int it,
                                                         const double *__restrict__ partials, int np,
                                                         double *__restrict__ pq) {
-  if (st->done) return;
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (ended(st, lead)) return;
   constexpr int V = chunk_entries<T>(), NC = 8 / V;
   typedef T VecT __attribute__((ext_vector_type(V)));
   const unsigned H = nl + 1, g = blockIdx.x * kBlock + threadIdx.x;
@@ -93,7 +104,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A,
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   T b = T(0);
   if (it > 0) {
     const Test t = test_of(st, partials, np);
@@ -164,10 +174,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_update(T *__restrict__ x, T *_
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   if (lead) st->pz = pz;
   if (pz != pz || pz == 0.0) {
-    if (lead) {
-      st->status = pz != pz ? LFRIC_NAN : LFRIC_BREAKDOWN;
-      st->done = 1;
-    }
+    if (lead) st->status = pz != pz ? LFRIC_NAN : LFRIC_BREAKDOWN;
     return;
   }
   if (lead) st->alpha = alpha;
@@ -189,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_update(T *__restrict__ x, T *_
 // the test after `it` iterations, for the host's read (the next iteration's first kernel forms it again)
 __global__ __launch_bounds__(kBlock) void k_cg_w0_test(SolverState *st, int it, const double *__restrict__ partials,
                                                        int np) {
-  if (st->done) return;
+  if (ended(st, threadIdx.x == 0)) return;
   const Test t = test_of(st, partials, np);
   if (threadIdx.x == 0) record(st, t, it);
 }

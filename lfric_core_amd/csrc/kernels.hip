@@ -1612,8 +1612,11 @@ __global__ __launch_bounds__(kBlock) void k_finish(const double *__restrict__ pa
 
 // CG's update with the p.(A p) finish folded in: every block adds the npz partials of the apply
 // itself (reduce_partials: the same total in every block) and forms alpha = rz / pz; block 0
-// records it (and a NaN or zero pz, which stops the solve in every block alike).  par selects
-// the iteration's rz slot (the host counts the iterations it enqueues).
+// records it (and a NaN or zero pz, which stops the solve in every block alike).  It records that in
+// `status` alone, which nothing here reads, and k_cg_aypx_fold turns it into `done`: set here, `done` would
+// be read by the later waves of blocks whose earlier waves started without it, and such a block would
+// add an incomplete pz and step x with it.  par selects the iteration's rz slot (the host counts the
+// iterations it enqueues).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cg_update_fold(T *__restrict__ x, T *__restrict__ r, T *__restrict__ z,
                                                            const T *__restrict__ p, const T *__restrict__ diag,
@@ -1628,7 +1631,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_fold(T *__restrict__ x, T 
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       st->pz = pz;
       st->status = pz != pz ? LFRIC_NAN : LFRIC_BREAKDOWN;
-      st->done = 1;
     }
     return;
   }
@@ -1677,11 +1679,14 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cg_aypx_fold(T *__restrict__ p, const T *__restrict__ z, long long n,
                                                          SolverState *st, const double *__restrict__ partials,
                                                          int nblocks, int par) {
-  if (st->done) return;
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (st->done || st->status) {  // the update met a NaN or zero p.(A p)
+    if (lead) st->done = 1;
+    return;
+  }
   double tot[2];
   reduce_partials<2>(partials, nblocks, tot);
   const double rn = sqrt(tot[0]);
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   if (rn != rn) {
     if (lead) {
       st->iter += 1;

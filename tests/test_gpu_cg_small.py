@@ -51,3 +51,20 @@ def test_ends_of_a_solve(hip):
     b = hip.FieldVector(fs).fill_uniform(1, 3)
     res, _ = _cg(hip, op, b, hip.R64, 1, r_tol=1e-12, a_tol=0.0, max_iter=3)
     assert res.status == 1 and res.iterations == 3
+
+
+@pytest.mark.parametrize("prec", ["R64", "R32"])
+@pytest.mark.parametrize("n,nl,order", [(2, 2, 0), (12, 20, 0), (25, 48, 0), (48, 60, 0), (6, 5, 1)])
+def test_breakdown_leaves_x_as_it_was(hip, n, nl, order, prec):
+    """A = 0: p.(A p) is 0 in the first iteration, which ends the solve before x is stepped, in the two-kernel
+    iteration and (vectors beyond 1.5 MB, order 1) in the separate kernels."""
+    P = getattr(hip, prec)
+    fs = hip.FunctionSpace.cubedsphere(n, nl, hip.W0, order)
+    op = hip.LmaOperator(fs, precision=P)
+    b, x = hip.FieldVector(fs, P).fill_uniform(n, 3), hip.FieldVector(fs, P).fill_uniform(nl, 4)
+    before = x.export_raw()
+    cg = hip.ConjugateGradient(op, hip.NullPreconditioner(), 1e-8, 0.0, 50)
+    with pytest.raises(hip.LfricError):
+        cg.apply(x, b)
+    assert cg.result.status == 3 and cg.result.iterations == 0
+    np.testing.assert_array_equal(x.export_raw(), before)
