@@ -67,7 +67,7 @@ int lfric_set_stream(void *stream);
 /* Time work on the library stream with HIP events: start, then stop returns milliseconds. */
 int lfric_timer_start(void);
 int lfric_timer_stop(double *ms);
-/* Bytes of device memory held by live handles. */
+/* Bytes of device memory held by live handles (buffers kept between batches: lfric_batch_kept_bytes). */
 long long lfric_device_bytes(void);
 /* LMA apply used inside the solvers: 0 the colour-ordered scatter (4 launches per apply),
  * 1 the gather form (one launch; in CG it also forms p.(A p)).  Default 1. */
@@ -517,6 +517,12 @@ int lfric_batch_config(lfric_batch *b, int use_graph, int block, int grid_mult);
 int lfric_batch_set_apply(lfric_batch *b, int form);
 int lfric_batch_stats(const lfric_batch *b, long long *iterations, int *block, int *grid_mult, int *ntiles);
 void lfric_batch_destroy(lfric_batch *b);
+/* Device buffers of destroyed batches and removed problems are kept for the next batches, at most 1 GiB
+ * in all, the longest-kept freed first beyond that.  They are no live handle's, so lfric_device_bytes does
+ * not count them: kept_bytes does.  release_kept frees them and returns their bytes; the library does so
+ * itself when one of its allocations fails. */
+long long lfric_batch_kept_bytes(void);
+long long lfric_batch_release_kept(void);
 
 #ifdef __cplusplus
 }

@@ -167,6 +167,8 @@ SIGNATURES = {
     "lfric_batch_stats": (_I, [_VP, ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(_I), ctypes.POINTER(_I),
                                ctypes.POINTER(_I)]),
     "lfric_batch_destroy": (None, [_VP]),
+    "lfric_batch_kept_bytes": (ctypes.c_longlong, []),
+    "lfric_batch_release_kept": (ctypes.c_longlong, []),
 }
 
 _lib = None

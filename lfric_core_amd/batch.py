@@ -50,6 +50,17 @@ def build_problem(n, nl, order, nrhs, seed, scaled=False, copies=True, fp64_copi
     return dict(fs=fs, op64=op64, op32=op32, d32=d32, b=b, x=x, nrhs=nrhs, key=(n, nl, order, nrhs, seed))
 
 
+def kept_bytes():
+    """Device bytes kept from destroyed batches for the next ones (at most 1 GiB; in no handle's
+    device_bytes)."""
+    return lib().lfric_batch_kept_bytes()
+
+
+def release_kept():
+    """Free the buffers kept for the next batches; their bytes."""
+    return lib().lfric_batch_release_kept()
+
+
 @dataclass
 class BatchProblem:
     """One problem of a batch: FP64 and FP32 copies of a square LMA operator, its Jacobi

@@ -34,7 +34,7 @@ int dmalloc(void **p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 64;
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && batch_buffers_release()) {
+  if (e != hipSuccess && batch_buffers_release() > 0) {
     (void)hipGetLastError();
     e = hipMalloc(p, bytes);
   }

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <deque>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -611,16 +612,26 @@ namespace {
 
 constexpr double kEps = 2.220446049250313e-16;
 
-// Device buffers of destroyed batches and removed problems, kept for the next of the same size: a program
-// that solves one batch after another spent 4 of 23 ms (8 problems) in hipMalloc and hipFree.  At most 1 GiB in
-// all (kept buffers count as free, not as held by live handles), given back when an allocation of the library
-// fails (batch_buffers_release).  Only idle buffers are put: their owners wait for the device first.
+// Device buffers of destroyed batches and removed problems, kept for the next: a program that solves one batch
+// after another spent 4 of 23 ms (8 problems) in hipMalloc and hipFree.  Buffers come in size classes, eight
+// to a factor of two (at most 1/8 more than asked for), so that batches of similar sizes share them.  At most
+// 1 GiB in all; beyond that the longest-kept go, so sizes that do not recur leave again.  Kept buffers are no
+// live handle's (lfric_device_bytes): lfric_batch_kept_bytes counts them and lfric_batch_release_kept frees
+// them, as does an allocation of the library that fails.  Only idle buffers are put: their owners wait for the
+// device first, and a buffer whose work may still run is freed instead (hipFree waits for it).
 std::mutex g_buf_mu;
-std::vector<std::pair<void *, size_t>> g_buf;
+std::deque<std::pair<void *, size_t>> g_buf;  // longest-kept first
 size_t g_buf_bytes = 0;
 constexpr size_t kBufMax = size_t{1} << 30;
 
+size_t buf_class(size_t bytes) {
+  size_t step = 64;
+  while (step * 16 < bytes) step *= 2;
+  return std::max<size_t>((bytes + step - 1) / step * step, 64);
+}
+
 int buf_get(void **p, size_t bytes) {
+  bytes = buf_class(bytes);
   {
     std::lock_guard<std::mutex> lk(g_buf_mu);
     for (size_t i = 0; i < g_buf.size(); ++i)
@@ -635,23 +646,30 @@ int buf_get(void **p, size_t bytes) {
   return dmalloc(p, bytes);
 }
 
+void buf_free(void *p, size_t bytes) { dfree(p, buf_class(bytes)); }
+
 void buf_put(void *p, size_t bytes) {
   if (!p) return;
+  bytes = buf_class(bytes);
+  if (bytes > kBufMax) return dfree(p, bytes);
+  std::vector<void *> out;
   {
     std::lock_guard<std::mutex> lk(g_buf_mu);
-    if (bytes > 0 && g_buf_bytes + bytes <= kBufMax) {
-      g_buf.emplace_back(p, bytes);
-      g_buf_bytes += bytes;
-      ctx().bytes -= static_cast<long long>(bytes);
-      return;
+    while (g_buf_bytes + bytes > kBufMax) {
+      out.push_back(g_buf.front().first);
+      g_buf_bytes -= g_buf.front().second;
+      g_buf.pop_front();
     }
+    g_buf.emplace_back(p, bytes);
+    g_buf_bytes += bytes;
+    ctx().bytes -= static_cast<long long>(bytes);
   }
-  dfree(p, bytes);
+  for (void *q : out) (void)hipFree(q);
 }
 
 int ensure(void **p, size_t &cap, size_t need, size_t elem) {
   if (need <= cap && *p) return LFRIC_OK;
-  dfree(*p, cap * elem);
+  buf_free(*p, cap * elem);
   *p = nullptr;
   cap = 0;
   const size_t c = std::max<size_t>(need, 16) * 2;
@@ -721,14 +739,14 @@ int alloc_state(lfric_batch &B, int nr, int *scal0) {
     RhsDev *d = nullptr, *h = nullptr;
     if (int rc = buf_get(reinterpret_cast<void **>(&d), cap * sizeof(RhsDev))) return rc;
     if (hipHostMalloc(reinterpret_cast<void **>(&h), cap * sizeof(RhsDev), hipHostMallocDefault) != hipSuccess) {
-      dfree(d, cap * sizeof(RhsDev));
+      buf_free(d, cap * sizeof(RhsDev));
       return fail(LFRIC_E_NOMEM, "pinned host state");
     }
     if (B.used_state) {
       LF_HIP(hipMemcpyAsync(d, B.d_state, B.used_state * sizeof(RhsDev), hipMemcpyDeviceToDevice, cur_stream()));
       LF_HIP(hipStreamSynchronize(cur_stream()));
     }
-    dfree(B.d_state, B.cap_state * sizeof(RhsDev));
+    buf_free(B.d_state, B.cap_state * sizeof(RhsDev));
     if (B.h_state) (void)hipHostFree(B.h_state);
     B.d_state = d;
     B.h_state = h;
@@ -1133,10 +1151,12 @@ int refine_all(lfric_batch &B, const std::vector<Problem *> &ps) {
   return LFRIC_OK;
 }
 
-void free_problem(lfric_batch &B, Problem &p) {
-  buf_put(p.d, p.bytes32);
-  buf_put(p.r64, p.bytes64);
-  buf_put(p.zs, p.zs_bytes);
+// idle: nothing that was enqueued still uses the problem's buffers
+void free_problem(lfric_batch &B, Problem &p, bool idle) {
+  const auto give = idle ? buf_put : buf_free;
+  give(p.d, p.bytes32);
+  give(p.r64, p.bytes64);
+  give(p.zs, p.zs_bytes);
   p.d = nullptr;
   p.r64 = nullptr;
   p.zs = nullptr;
@@ -1187,15 +1207,17 @@ int run_rounds(lfric_batch &B, int rounds, int *nactive) {
 
 }  // namespace
 
-bool batch_buffers_release() {
-  std::vector<std::pair<void *, size_t>> all;
+long long batch_buffers_release() {
+  std::deque<std::pair<void *, size_t>> all;
+  long long bytes = 0;
   {
     std::lock_guard<std::mutex> lk(g_buf_mu);
     all.swap(g_buf);
+    bytes = static_cast<long long>(g_buf_bytes);
     g_buf_bytes = 0;
   }
   for (auto &b : all) (void)hipFree(b.first);
-  return !all.empty();
+  return bytes;
 }
 
 }  // namespace lfric
@@ -1253,11 +1275,11 @@ int lfric_batch_add(lfric_batch *B, const lfric_op *A64, const lfric_op *A32, co
   p->scal0 = -1;
   if (int rc = buf_get(reinterpret_cast<void **>(&p->d), p->bytes32)) return rc;
   if (int rc = buf_get(reinterpret_cast<void **>(&p->r64), p->bytes64)) {
-    free_problem(*B, *p);
+    free_problem(*B, *p, true);
     return rc;
   }
   if (int rc = alloc_state(*B, nr, &p->scal0)) {
-    free_problem(*B, *p);
+    free_problem(*B, *p, true);
     return rc;
   }
   p->r = p->d + p->n;
@@ -1270,7 +1292,7 @@ int lfric_batch_add(lfric_batch *B, const lfric_op *A64, const lfric_op *A32, co
   // the gather lists of the space (built once per space)
   if (!A32->to->d_gcol)
     if (int rc = launch_lma_apply_mrhs(A64, x->d, p->r64, nr, LFRIC_MRHS_GATHER)) {
-      free_problem(*B, *p);
+      free_problem(*B, *p, false);
       return rc;
     }
   p->id = B->next_id++;
@@ -1330,7 +1352,7 @@ int lfric_batch_remove(lfric_batch *B, int id) {
     if (B->probs[i]->id == id) {
       if (B->probs[i]->inner_running) B->dirty = true;
       LF_HIP(hipDeviceSynchronize());  // as in lfric_batch_destroy
-      free_problem(*B, *B->probs[i]);
+      free_problem(*B, *B->probs[i], true);
       B->probs.erase(B->probs.begin() + static_cast<long>(i));
       return LFRIC_OK;
     }
@@ -1400,20 +1422,29 @@ int lfric_batch_stats(const lfric_batch *B, long long *iterations, int *block, i
   return LFRIC_OK;
 }
 
+long long lfric_batch_kept_bytes(void) {
+  std::lock_guard<std::mutex> lk(g_buf_mu);
+  return static_cast<long long>(g_buf_bytes);
+}
+
+long long lfric_batch_release_kept(void) { return batch_buffers_release(); }
+
 void lfric_batch_destroy(lfric_batch *B) {
   if (!B) return;
-  (void)hipDeviceSynchronize();  // the buffers go to the next batch idle, whatever stream it uses
-  for (auto &u : B->probs) free_problem(*B, *u);
+  // the buffers go to the next batch idle, whatever stream it uses; freed if the wait fails
+  const bool idle = hipDeviceSynchronize() == hipSuccess;
+  const auto give = idle ? buf_put : buf_free;
+  for (auto &u : B->probs) free_problem(*B, *u, idle);
   drop_graph(*B);
-  buf_put(B->d_state, B->cap_state * sizeof(RhsDev));
+  give(B->d_state, B->cap_state * sizeof(RhsDev));
   if (B->h_state) (void)hipHostFree(B->h_state);
-  buf_put(B->d_desc, B->cap_desc * sizeof(ProbDev));
-  buf_put(B->d_tile0, B->cap_tile0 * sizeof(int));
-  buf_put(B->d_vtile0, B->cap_vtile0 * sizeof(int));
-  buf_put(B->d_partials, B->cap_partials * sizeof(double));
+  give(B->d_desc, B->cap_desc * sizeof(ProbDev));
+  give(B->d_tile0, B->cap_tile0 * sizeof(int));
+  give(B->d_vtile0, B->cap_vtile0 * sizeof(int));
+  give(B->d_partials, B->cap_partials * sizeof(double));
   dfree(B->d_scratch, sizeof(double) * kSlot * B->scratch_slots);
   dfree(B->d_counter, sizeof(unsigned int) * kCounters);
-  buf_put(B->d_ctile0, B->cap_ctile0 * sizeof(int));
+  give(B->d_ctile0, B->cap_ctile0 * sizeof(int));
   if (B->h_scratch) (void)hipHostFree(B->h_scratch);
   delete B;
 }

@@ -47,8 +47,8 @@ hipStream_t cur_stream();
 int require_init();
 int dmalloc(void **p, size_t bytes);
 void dfree(void *p, size_t bytes);
-// free the buffers that destroyed batches left for the next (batch.hip); whether there were any
-bool batch_buffers_release();
+// free the buffers that destroyed batches left for the next (batch.hip); their bytes
+long long batch_buffers_release();
 
 // ---- mesh topology (host) ---------------------------------------------------------------
 // Serial-partition extruded cubed-sphere base-layer connectivity.

@@ -136,11 +136,12 @@ def test_batch_copy_forms_equal_colour_and_gather_forms(hip, orc):
 
 def test_batches_one_after_another_reuse_their_buffers(hip):
     """A second batch of the same problems, after the first is destroyed, gets the first one's buffers: the
-    same results bit for bit (nothing is read before it is written), and no device memory is held by
-    either afterwards."""
-    from lfric_core_amd.batch import Batch, build_problem
+    same results bit for bit (nothing is read before it is written).  Afterwards no handle holds device memory;
+    what is kept is counted, does not grow from batch to batch, and is given back on request."""
+    from lfric_core_amd.batch import Batch, build_problem, kept_bytes, release_kept
+    release_kept()
     probs = [build_problem(4, 5, 0, 4, 1), build_problem(3, 4, 1, 2, 2), build_problem(5, 3, 1, 1, 3)]
-    held, out = [hip.device_bytes()], []
+    held, kept, out = [hip.device_bytes()], [], []
     for _ in range(3):
         bt = Batch(r_tol=1e-8, a_tol=0.0, max_iter=500, check_every=8)
         for p in probs:
@@ -149,9 +150,45 @@ def test_batches_one_after_another_reuse_their_buffers(hip):
         bt.solve()
         bt.close()
         held.append(hip.device_bytes())
+        kept.append(kept_bytes())
         out.append([p["x"].export_field() for p in probs])
     # the first batch may build its operators' lists; after it nothing grows
     assert held[1] == held[2] == held[3]
+    assert 0 < kept[0] == kept[1] == kept[2]
+    assert release_kept() == kept[2] and kept_bytes() == 0 == release_kept()
     for later in out[1:]:
         for a, b in zip(out[0], later):
             np.testing.assert_array_equal(a, b)
+
+
+def test_kept_buffers_are_bounded_and_follow_changing_sizes(hip):
+    """Batches whose sizes change: nearby sizes share buffers, the list stays within 1 GiB, and sizes that
+    do not recur make room for those of the latest batch.  (Problems are added and not solved: only their
+    buffers matter here.)"""
+    from lfric_core_amd.batch import Batch, kept_bytes, release_kept
+    release_kept()
+
+    def add(n, nl, nrhs, count):
+        fs = hip.FunctionSpace.cubedsphere(n, nl)
+        op64, op32 = hip.LmaOperator(fs), hip.LmaOperator(fs, precision=hip.R32)
+        d32, x, b = hip.FieldVector(fs, hip.R32), hip.FieldVector(fs, hip.R64, nrhs), hip.FieldVector(fs, hip.R64, nrhs)
+        bt = Batch()
+        for _ in range(count):
+            bt.add(op64, op32, d32, x, b)
+        taken = kept_bytes()  # while the batch holds its own
+        bt.close()
+        return taken
+
+    add(12, 20, 4, 2)
+    first = kept_bytes()
+    assert add(12, 20, 4, 2) == 0 and kept_bytes() == first
+    # 24 bytes a dof and right-hand side: a problem of C64x60 with 8 right-hand sides takes 288 MB
+    limit = 1 << 30
+    for nrhs in (8, 4, 8):
+        add(64, 60, nrhs, 5)
+        assert limit // 2 < kept_bytes() <= limit
+        assert add(64, 60, nrhs, 3) <= limit - 3 * 24 * nrhs * (6 * 64 * 64 + 2) * 61  # all 3 from the list
+    # a size within the same class (one level in 60 more or less) takes the same buffers
+    before = kept_bytes()
+    assert add(64, 59, 8, 1) <= before - 24 * 8 * (6 * 64 * 64 + 2) * 60
+    assert release_kept() <= limit and kept_bytes() == 0
