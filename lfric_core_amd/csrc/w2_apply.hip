@@ -16,21 +16,22 @@ namespace lfric {
 namespace {
 
 // Each cell position's neighbour across its side faces W, S, E, N as neighbour position * 8 + the face's
-// number there, -1 where there is none.  False where a side face has more than two cells.
+// number there, -1 where there is none.  False where the kernels below do not hold, as a caller's dofmap may
+// have it: a side face of more than two cells, or a bottom-face column (dof 4) that other faces share.
 bool w2_neighbours(const FunctionSpace &f, std::vector<int4> &tab) {
   struct Item {
     int base, pos, df;
   };
   std::vector<Item> items;
-  items.reserve(static_cast<size_t>(f.ncells) * 4);
+  items.reserve(static_cast<size_t>(f.ncells) * 5);
   for (int p = 0; p < f.ncells; ++p)
-    for (int d = 0; d < 4; ++d) items.push_back({f.dofmap[static_cast<size_t>(f.cell_of_pos[p]) * 6 + d], p, d});
+    for (int d = 0; d < 5; ++d) items.push_back({f.dofmap[static_cast<size_t>(f.cell_of_pos[p]) * 6 + d], p, d});
   std::sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.base < b.base; });
   tab.assign(f.ncells, make_int4(-1, -1, -1, -1));
   for (size_t q = 1; q < items.size(); ++q) {
     const Item &a = items[q - 1], &b = items[q];
     if (a.base != b.base) continue;
-    if (q + 1 < items.size() && items[q + 1].base == b.base) return false;
+    if (a.df == 4 || b.df == 4 || (q + 1 < items.size() && items[q + 1].base == b.base)) return false;
     (&tab[a.pos].x)[a.df] = b.pos * 8 + b.df;
     (&tab[b.pos].x)[b.df] = a.pos * 8 + a.df;
   }
