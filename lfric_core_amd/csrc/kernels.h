@@ -92,7 +92,8 @@ bool mfma_apply_supported(const lfric_op *op);
 int batch_colour_form(const lfric_op *op);
 int launch_lma_transpose(const lfric_op *op, const void *x, void *y);
 // Each cell's side neighbours of a lowest-order W2 space, and (columns) the cells of its dof columns: no table,
-// with LFRIC_OK, for other spaces and where a side face has more than two cells.  Over them: the apply of a
+// with LFRIC_OK, for other spaces, where a side face has more than two cells and where bottom-face columns are
+// shared.  Over them: the apply of a
 // square operator, with the gather form's sums or (colour) the colour-ordered form's, bit for bit, and enforce_bc
 // with bc; the transpose of a 1 x 6 operator (both always faster than the kernels without tables, which stay
 // for other spaces); and the Helmholtz composite in one kernel: build_helm_table sets hcol_state, 1 where

@@ -1289,7 +1289,8 @@ __global__ __launch_bounds__(kBlock) void k_transpose_colour(const T *__restrict
 }
 
 // ---- Helmholtz composite y = M3 x + tau D diag(M2)^-1 D^T x in two kernels ------------------
-// For meshes without the neighbour table of the one-kernel form (w2_apply.hip).  (W3 <- W2 lowest order: D holds 1 x 6 per element, M3 1 x 1.)  The first is the transpose in
+// For dofmaps without the neighbour table of the one-kernel form (w2_apply.hip): side faces of three cells, shared
+// bottom-face columns.  (W3 <- W2 lowest order: D holds 1 x 6 per element, M3 1 x 1.)  The first is the transpose in
 // gather form with the division by m2 folded in: W2 dof (column, level m) adds its cells'
 // contributions in colour order, the first written and the rest added, each the colour-
 // ordered transpose's chain (row of layer m, then the top partner's of layer m-1), then divides
@@ -2181,7 +2182,7 @@ int launch_op_convert(const lfric_op *src, lfric_op *dst) {
 
 // ---- operator apply dispatch ---------------------------------------------------------------
 template <typename T, int A_, int B_>
-static void launch_colour(RoleKind rk, int grid, const lfric_op *op, size_t S, const T *x, T *y, const FunctionSpace &to,
+static int launch_colour(RoleKind rk, int grid, const lfric_op *op, size_t S, const T *x, T *y, const FunctionSpace &to,
                           const FunctionSpace &from, const uint32_t *first, int pos0, int npos, const int *d_skip) {
   const int nl = to.nlayers;
   const T *Ad = static_cast<const T *>(op->d);
@@ -2191,8 +2192,8 @@ static void launch_colour(RoleKind rk, int grid, const lfric_op *op, size_t S, c
         LAUNCH((k_lma_colour<T, A_, B_, RolesW0K0>), grid, Ad, S, to.d_ebase, x, y, to.d_map, from.d_map, first, pos0, npos, nl,
                RolesW0K0{}, d_skip, op->xwin);
       break;
-    case RoleKind::W0K1:  // launch_colour_rows27
-      break;
+    case RoleKind::W0K1:  // square ones take launch_colour_rows27
+      return fail(LFRIC_E_UNSUPPORTED, "lma_apply: unsupported (ndf_to, ndf_from)");
     case RoleKind::W2K0:
       if constexpr (A_ == 6)
         LAUNCH((k_lma_colour<T, A_, B_, RolesW2K0>), grid, Ad, S, to.d_ebase, x, y, to.d_map, from.d_map, first, pos0, npos, nl,
@@ -2206,6 +2207,7 @@ static void launch_colour(RoleKind rk, int grid, const lfric_op *op, size_t S, c
       LAUNCH((k_lma_colour<T, A_, B_, RolesRuntime>), grid, Ad, S, to.d_ebase, x, y, to.d_map, from.d_map, first, pos0, npos, nl,
              RolesRuntime{roles_of(to)}, d_skip, op->xwin);
   }
+  return LFRIC_OK;
 }
 
 template <typename T>
@@ -2223,7 +2225,7 @@ static int apply_colours_t(const lfric_op *op, const T *x, T *y, const int *d_sk
     const int grid = grid_for(static_cast<long long>(npos) * (nl + 1));
 #define LMA_CASE(A, B)                                                                              \
   if (to.ndf == A && from.ndf == B) {                                                              \
-    launch_colour<T, A, B>(rk, grid, op, S, x, y, to, from, to.d_first, pos0, npos, d_skip);    \
+    if (int rc = launch_colour<T, A, B>(rk, grid, op, S, x, y, to, from, to.d_first, pos0, npos, d_skip)) return rc; \
     continue;                                                                                       \
   }
     LMA_CASE(8, 8)

@@ -1,5 +1,6 @@
-// One point of the lowest-order W0 apply from its column's table entry, shared by the apply and the conjugate
-// gradient's.
+// The table entry of a lowest-order W0 dof column, and one point of the apply from it.  The small conjugate
+// gradient's apply (cg_w0.hip) reads the same entries and states the same gather chain with its loads of z and
+// the old p placed for it; tests hold the two to the same bits.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -73,12 +73,12 @@ def test_helmholtz_apply_parity(hip, orc, n, nl):
 
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("n,nl", [(4, 3), (5, 7), (12, 10)])
-def test_helmholtz_two_kernel_apply_equals_the_kernel_chain(hip, orc, n, nl, precision):
-    """The Helmholtz composite's two-kernel apply (transpose in gather form with the division,
-    over the composite's copy of D in transpose-gather order, then divergence, M3 and the axpy
-    in one kernel) equals the chain of separate applies - colour-ordered transpose, division by
-    diag(M2), divergence, M3, y += tau t - bit for bit; after D's or M3's entries are
-    rewritten the composite's copies follow them."""
+def test_helmholtz_one_kernel_apply_equals_the_kernel_chain(hip, orc, n, nl, precision):
+    """The Helmholtz composite's one-kernel apply (each cell and layer forms the gradient of its six
+    faces itself, over the composite's copy of D and M3) equals the chain of separate applies -
+    transpose, division by diag(M2), divergence, M3, y += tau t - bit for bit; after D's or M3's
+    entries are rewritten the composite's copy follows them.  (The two-kernel form, for dofmaps without
+    the neighbour table: tests/test_gpu_w2_table.py.)"""
     tau = 0.5
     w2, w3, H, (M2, D, M3, m2d) = _helmholtz(hip, orc, n, nl, precision, tau)
     x = hip.FieldVector(w3, precision).fill_uniform(3, 3)
