@@ -3,7 +3,9 @@ sizes that leave partial blocks and partial groups of blocks, on one and on seve
 
 * Against the element matrices and the dofmap in numpy, FP64: every output is a sum of at most 4 cells' fma
   chains of 27 terms (two for a dof shared by layers), so it is within (27 + 8) eps of |A| |x|.
-* Several right-hand sides equal the one-right-hand-side apply column by column, bit for bit."""
+* Several right-hand sides equal the one-right-hand-side apply column by column, bit for bit; also on both
+  sides of the colour sizes (16384 and 32768 units) where the split of a unit's rows changes and where one
+  thread a unit takes over, and in the automatic choice (for 8 FP64 right-hand sides the gather form's bits)."""
 import numpy as np
 import pytest
 
@@ -37,3 +39,30 @@ def test_order1_colour_apply(hip, n, nl, prec):
         ym.set_scalar(-3.0)
         op.apply_mrhs(xm, ym, 2)
         np.testing.assert_array_equal(ym.export_raw().reshape(fs.undf, nr), np.stack(cols[:nr], 1))
+
+
+@pytest.mark.parametrize("prec", ["R64", "R32"])
+@pytest.mark.parametrize("nl,units", [(17, 15552), (18, 16416), (36, 31968), (37, 32832)])
+def test_order1_colour_apply_beside_the_split_limits(hip, nl, units, prec):
+    P, T = getattr(hip, prec), np.float64 if prec == "R64" else np.float32
+    fs = hip.FunctionSpace.cubedsphere(24, nl, hip.W0, 1)
+    assert int(fs.colouring()[0].max()) * (nl + 1) == units
+    op = hip.LmaOperator(fs).generate_spd(nl)
+    op = op if P == hip.R64 else op.convert(P)
+    X = np.random.default_rng(nl).uniform(-1, 1, (fs.undf, 8)).astype(T)
+    x, y = hip.FieldVector(fs, P), hip.FieldVector(fs, P)
+    cols = []
+    for r in range(8):
+        op.apply(x.import_raw(X[:, r].copy()), y)
+        cols.append(y.export_raw())
+    for nr in (2, 4, 8):
+        xm, ym = hip.FieldVector(fs, P, nr).import_raw(X[:, :nr].ravel()), hip.FieldVector(fs, P, nr)
+        for variant in (2, 0):
+            ym.set_scalar(-3.0)
+            op.apply_mrhs(xm, ym, variant)
+            got = ym.export_raw().reshape(fs.undf, nr)
+            if variant == 0 and nr == 8 and prec == "R64":
+                op.apply_mrhs(xm, ym, 1)
+                np.testing.assert_array_equal(got, ym.export_raw().reshape(fs.undf, nr))
+            else:
+                np.testing.assert_array_equal(got, np.stack(cols[:nr], 1))
