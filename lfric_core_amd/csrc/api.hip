@@ -273,7 +273,7 @@ struct CgArgs {
 // then reads the device state once; kernels of iterations past convergence return at once.
 // Byte offsets of r, z, p and the p.Ap partials inside the allocation-free CG's scratch array:
 // each piece starts on a 256-byte boundary.  Returns the bytes used.
-// The small CG's q and second p follow them (it takes vectors of at most 1.5 MB, so they fit).
+// The small CG's q and second p follow them (it takes vectors of at most 1 MB, so they fit).
 static size_t cg_scratch_layout(size_t vb, int pz_blocks, size_t off[6]) {
   const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   off[0] = 0;

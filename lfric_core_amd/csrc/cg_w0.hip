@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_test(SolverState *st, int it, 
   if (threadIdx.x == 0) record(st, t, it);
 }
 
-constexpr int kAheadBlocks = 256;  // compute units
+constexpr int kUnits = 256;  // compute units
 
 template <typename T>
 int iteration_t(const lfric_op *op, void *const (&v)[6], const T *diag, SolverState *st, int it) {
@@ -213,7 +213,7 @@ int iteration_t(const lfric_op *op, void *const (&v)[6], const T *diag, SolverSt
   // loads ahead while all blocks are resident at once (a wave on a SIMD in FP64, two in FP32).  Solves without -> with,
   // FP64: C12x20 (72 blocks) 283 -> 257 us, C20x25 (244) 321 -> 288, C24x30 (419) 423 -> 438; FP32: C12x20 167 -> 149,
   // C24x36 (500) 216 -> 191
-  auto apply = nb <= (sizeof(T) == 4 ? 2 : 1) * kAheadBlocks ? k_cg_w0_apply<T, true> : k_cg_w0_apply<T, false>;
+  auto apply = nb <= (sizeof(T) == 4 ? 2 : 1) * kUnits ? k_cg_w0_apply<T, true> : k_cg_w0_apply<T, false>;
   hipLaunchKernelGGL(apply, dim3(nb), dim3(kBlock), 0, cur_stream(), static_cast<const T *>(op->d), op->gs,
                      static_cast<const W0Col *>(f.d_w0tab), z, it > 0 ? pold : z, pnew, q, f.w0tab_cols, f.nlayers, st,
                      it, part, nb, pq);
@@ -225,13 +225,15 @@ int iteration_t(const lfric_op *op, void *const (&v)[6], const T *diag, SolverSt
 
 }  // namespace
 
-// Vectors of up to 1.5 MB: there the launches that it saves outweigh reading two vectors where the apply of three
-// kernels reads one.  FP64 solves of 12-13 iterations, three kernels -> two: 18186 dofs 355 -> 250 us, 107198 445 ->
-// 407, 176358 530 -> 497; 329522 706 -> 779.  FP32, 8 iterations: 18186 212 -> 148, 329522 340 -> 313; 552238 422 -> 491.
+// Up to the blocks that are resident at once without loads ahead (two on a compute unit in FP64, three in FP32).  There
+// the launches that it saves outweigh reading two vectors where the apply of three kernels reads one; the first
+// block beyond takes a second round of the whole kernel.  16 iterations, three kernels -> two, FP64: 18186 dofs 367 ->
+// 262 us, 107198 504 -> 475, 127946 (500 blocks) 530 -> 502, 138320 (541) 557 -> 610, 176358 617 -> 717; FP32: 18186
+// 357 -> 253, 176358 468 -> 440, 192946 (754 blocks) 485 -> 452, 211770 (828) 512 -> 588, 374906 631 -> 704.
 bool cg_w0_usable(const lfric_op *op) {
   const FunctionSpace &f = *op->to;
   return f.d_w0tab && op->to == op->from && !op->sym && f.undf == f.w0tab_cols * (f.nlayers + 1) &&
-         static_cast<long long>(f.undf) * (op->precision == LFRIC_R64 ? 8 : 4) <= 1500000;
+         grid_for(f.undf) <= (op->precision == LFRIC_R64 ? 2 : 3) * kUnits;
 }
 
 int launch_cg_w0_iteration(const lfric_op *op, void *const (&v)[6], const void *diag, SolverState *st, int it) {

@@ -144,7 +144,7 @@ int launch_cg_finish_pz(const double *partials, int nblocks, SolverState *st, in
 // one iteration over the element layout of a lowest-order W0 operator in two kernels, for small problems: v =
 // x, r, z, q, and the two buffers of p.  The first kernel of an iteration tests the one before, so the host's reads
 // follow launch_cg_w0_test; cg_w0.hip
-constexpr int kCgW0Blocks = 2048;  // at most, of 256 dofs (FP32 vectors of 1.5 MB take 1465): 3 partials each
+constexpr int kCgW0Blocks = 768;  // at most, of 256 dofs (FP32; cg_w0_usable): 3 partials each
 bool cg_w0_usable(const lfric_op *op);
 int launch_cg_w0_iteration(const lfric_op *op, void *const (&v)[6], const void *diag, SolverState *st, int it);
 int launch_cg_w0_test(const lfric_op *op, SolverState *st, int it);

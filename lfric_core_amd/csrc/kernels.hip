@@ -1109,31 +1109,35 @@ __device__ inline double sym_gather_point(long long t, const T *__restrict__ z, 
   return to_d(acc) * to_d(x[static_cast<size_t>(ci.x) + m]);
 }
 
-// kSymPoints points per thread, kBlock apart: over the int4 table all their loads are requested before any
-// is added (C96x70 FP32: 21.3 us a point at a time, 15.6 us).
+// POINTS (1 or kSymPoints) points per thread, kBlock apart: with several, over the int4 table, all their loads are
+// requested before any is added.  Several from kSymPointsMin points (8 blocks a compute unit at one point a thread);
+// fewer leave units without a block.  Whole apply, one -> four points, FP32: 47678 points 7.7 -> 8.2 us, 374906 15.5 ->
+// 16.0, 569282 23.3 -> 23.1, 1147898 42.5 -> 40.5, 3926158 (C96x70) 134.3 -> 128.5 (its second phase 21.3 -> 15.6); FP64: 47678
+// 8.4 -> 9.6, 176358 15.0 -> 15.7, 649822 45.1 -> 45.0, 3926158 249.7 -> 247.9.
 constexpr int kSymPoints = 4;
-template <typename T>
+constexpr long long kSymPointsMin = 524288;
+template <typename T, int POINTS>
 __global__ __launch_bounds__(kBlock) void k_sym_gather(const T *__restrict__ z, const T *__restrict__ x,
                                                         T *__restrict__ y, const int2 *__restrict__ cols,
                                                         const int *__restrict__ off, const int *__restrict__ ent,
                                                         const int4 *__restrict__ zu, int ncols, int nl, const int *skip,
                                                         int xwin) {
   if (skip && *skip) return;
-  const long long t0 = static_cast<long long>(xcd_block(blockIdx.x, gridDim.x, xwin)) * kBlock * kSymPoints + threadIdx.x;
+  const long long t0 = static_cast<long long>(xcd_block(blockIdx.x, gridDim.x, xwin)) * kBlock * POINTS + threadIdx.x;
   const unsigned H = nl + 1;
   const long long total = static_cast<long long>(ncols) * H;
-  if (!zu || total >= (1LL << 31)) {
-    for (int e = 0; e < kSymPoints; ++e)
+  if (POINTS == 1 || !zu || total >= (1LL << 31)) {
+    for (int e = 0; e < POINTS; ++e)
       (void)sym_gather_point<T>(t0 + e * kBlock, z, x, y, cols, off, ent, zu, ncols, nl);
     return;
   }
-  T v[kSymPoints][4];
-  int4 us[kSymPoints];
-  int2 ci[kSymPoints];
-  unsigned m[kSymPoints];
-  bool ok[kSymPoints];
+  T v[POINTS][4];
+  int4 us[POINTS];
+  int2 ci[POINTS];
+  unsigned m[POINTS];
+  bool ok[POINTS];
 #pragma unroll
-  for (int e = 0; e < kSymPoints; ++e) {
+  for (int e = 0; e < POINTS; ++e) {
     const long long t = t0 + e * kBlock;
     ok[e] = t < total;
     const unsigned col = ok[e] ? static_cast<unsigned>(t) / H : 0;
@@ -1142,14 +1146,14 @@ __global__ __launch_bounds__(kBlock) void k_sym_gather(const T *__restrict__ z, 
     ci[e] = cols[col];
   }
 #pragma unroll
-  for (int e = 0; e < kSymPoints; ++e) {
+  for (int e = 0; e < POINTS; ++e) {
     ok[e] = ok[e] && (m[e] < H - 1 || ci[e].y);
     const int w[4] = {us[e].x, us[e].y, us[e].z, us[e].w};
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[e][q] = ok[e] && w[q] >= 0 ? z[static_cast<size_t>(w[q]) * H + m[e]] : T(0);
   }
 #pragma unroll
-  for (int e = 0; e < kSymPoints; ++e) {
+  for (int e = 0; e < POINTS; ++e) {
     const int w[4] = {us[e].x, us[e].y, us[e].z, us[e].w};
     T acc = v[e][0];
 #pragma unroll
@@ -2406,10 +2410,13 @@ static int launch_gather_r(const lfric_op *op, const T *x, T *y, R roles, Gather
       if (ex.partials)
         LAUNCH((k_sym_gather_dot<T>), kRedBlocks, static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff,
                to.d_gent, op->d_symzu, to.gather_ncols, to.nlayers, ex.partials, ex.skip, op->xwin);
-      else
-        LAUNCH((k_sym_gather<T>),
+      else if (static_cast<long long>(to.gather_ncols) * (to.nlayers + 1) >= kSymPointsMin)
+        LAUNCH((k_sym_gather<T, kSymPoints>),
                grid_for(static_cast<long long>(to.gather_ncols) * (to.nlayers + 1), kBlock * kSymPoints),
-               static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent,
+               static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent, op->d_symzu, to.gather_ncols,
+               to.nlayers, ex.skip, op->xwin);
+      else
+        LAUNCH((k_sym_gather<T, 1>), grid, static_cast<const T *>(op->symz), x, y, to.d_gcol, to.d_goff, to.d_gent,
                op->d_symzu, to.gather_ncols, to.nlayers, ex.skip, op->xwin);
       return LFRIC_OK;
     }

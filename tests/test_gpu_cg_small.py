@@ -1,8 +1,9 @@
 """Conjugate gradients in two kernels an iteration (small lowest-order W0 problems) against the form over the
 colour-ordered apply in separate kernels, whose sums run in another order: the same iterates up to rounding
 after a fixed number of iterations (the recurrences' error grows by the condition of B B^T + 0.1 I elements, below
-100: 1e4 eps of the norm), counts within one to a tolerance, and the ends of a solve.  Sizes of one block,
-several, a partial one, and both sides of the largest it takes (1.5 MB vectors)."""
+100: 1e4 eps of the norm), counts within one to a tolerance, and the ends of a solve.  Sizes of one block, several, a
+partial one, both sides of the loads ahead (256 and 512 blocks of 256 dofs, FP64 and FP32) and of the largest it
+takes (512 and 768 blocks), and beyond."""
 import numpy as np
 import pytest
 
@@ -21,7 +22,8 @@ def _cg(hip, op, b, P, form, **kw):
 
 
 @pytest.mark.parametrize("prec", ["R64", "R32"])
-@pytest.mark.parametrize("n,nl", [(2, 2), (3, 4), (5, 7), (12, 20), (25, 48), (25, 49), (32, 60)])
+@pytest.mark.parametrize("n,nl", [(2, 2), (3, 4), (5, 7), (12, 20), (20, 26), (20, 27), (24, 36), (24, 37),
+                                  (28, 40), (28, 41), (25, 48), (25, 49), (32, 60)])
 def test_two_kernel_iteration(hip, n, nl, prec):
     P, eps = (hip.R64, np.finfo(np.float64).eps) if prec == "R64" else (hip.R32, np.finfo(np.float32).eps)
     fs = hip.FunctionSpace.cubedsphere(n, nl)
@@ -57,7 +59,7 @@ def test_ends_of_a_solve(hip):
 @pytest.mark.parametrize("n,nl,order", [(2, 2, 0), (12, 20, 0), (25, 48, 0), (48, 60, 0), (6, 5, 1)])
 def test_breakdown_leaves_x_as_it_was(hip, n, nl, order, prec):
     """A = 0: p.(A p) is 0 in the first iteration, which ends the solve before x is stepped, in the two-kernel
-    iteration and (vectors beyond 1.5 MB, order 1) in the separate kernels."""
+    iteration and (beyond 512 or 768 blocks, order 1) in the separate kernels."""
     P = getattr(hip, prec)
     fs = hip.FunctionSpace.cubedsphere(n, nl, hip.W0, order)
     op = hip.LmaOperator(fs, precision=P)

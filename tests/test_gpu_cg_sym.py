@@ -9,6 +9,8 @@
   are scaled by 10^U(-2, 2): hundreds of FP32 iterations carry one rounding of alpha to another stopping
   point, so the products have to be those of the vectors themselves (p . (A p) of the gathered A p).  Up to
   2048 blocks of 256 dofs a dot's partial sums are the apply's.
+* The apply itself against the colour-ordered one, bit for bit, on both sides of the size (524288 points)
+  from which a thread of its second kernel takes several points.
 * The scaled mixed-precision solve against its refinement written out the same way, and its residual in
   the oracle's assembled matrix."""
 import numpy as np
@@ -149,3 +151,19 @@ def test_scaled_mixed_precision_solve(hip, orc, copy):
     S = orc.assembled_csr(m, orc.gen_spd(m.ndf, m.ncell_3d, 20, scaled=True))
     bb = b.export_field()
     assert np.linalg.norm(bb - S @ x.export_field()) <= 1e-8 * np.linalg.norm(bb)
+
+
+@pytest.mark.parametrize("prec", ["R64", "R32"])
+@pytest.mark.parametrize("nl,points", [(36, 511562), (37, 525388)])
+def test_apply_beside_the_several_points_limit(hip, nl, points, prec):
+    P = getattr(hip, prec)
+    fs = hip.FunctionSpace.cubedsphere(48, nl)
+    assert fs.undf == points
+    op = hip.LmaOperator(fs).generate_spd(nl)
+    op = op if P == hip.R64 else op.convert(P)
+    x, y, z = hip.FieldVector(fs, P).fill_uniform(1), hip.FieldVector(fs, P), hip.FieldVector(fs, P)
+    op.apply(x, y)
+    op.prepare_symmetric()
+    z.set_scalar(7.0)
+    hip.LinearOperator.from_lma(op).apply(x, z)
+    np.testing.assert_array_equal(z.export_raw(), y.export_raw())
