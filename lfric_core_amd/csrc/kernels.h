@@ -40,7 +40,8 @@ int launch_lma_apply(const lfric_op *op, const void *x, void *y, const int *d_sk
 // The gather lists of a lowest-order W0 space as one table entry per dof column (no table, with
 // LFRIC_OK, for other spaces and where a column has more than 4 cells), and the apply of a square
 // operator over it: the gather form's sums, or (colour) the colour-ordered form's, bit for bit;
-// w0_apply.hip.  The table is always the faster form, so there is no rule of sizes.
+// w0_apply.hip.  The table is the faster form from C4x5 to C96x70, colour-ordered by 1.2 to 4.7 times and gathered by 1.0
+// to 1.4, so there is no rule of sizes.
 int build_w0_table(FunctionSpace &f);
 int launch_w0_gather(const lfric_op *op, const void *x, void *y, bool colour, double *partials, const int *skip);
 // the space's gather lists, built on first use
@@ -95,9 +96,12 @@ int launch_lma_transpose(const lfric_op *op, const void *x, void *y);
 // with LFRIC_OK, for other spaces, where a side face has more than two cells and where bottom-face columns are
 // shared.  Over them: the apply of a
 // square operator, with the gather form's sums or (colour) the colour-ordered form's, bit for bit, and enforce_bc
-// with bc; the transpose of a 1 x 6 operator (both always faster than the kernels without tables, which stay
-// for other spaces); and the Helmholtz composite in one kernel: build_helm_table sets hcol_state, 1 where
-// launch_helm applies; w2_apply.hip
+// with bc; the transpose of a 1 x 6 operator; and the Helmholtz composite in one kernel: build_helm_table sets
+// hcol_state, 1 where launch_helm applies; w2_apply.hip.  The kernels without tables stay for other spaces.  From
+// C4x6 to C96x70 the tables' are the faster ones by 1.0 to 5 times in both types, but for FP32 mass matrices of 190 to
+// 256 MB (C56x70 to C64x70): where they still fit the last-level cache and launches no longer count,
+// reading the chunk that two rows share twice shows (a thread of the colours has both rows): C64x70 68 -> 76 us, C72x70
+// 101 -> 97.  That window is no reason for a branch: it closes as soon as other data passes through the cache.
 int build_w2_table(FunctionSpace &f, bool columns);
 int launch_w2_gather(const lfric_op *op, const void *x, void *y, bool colour, double *partials, const int *skip, int bc);
 int launch_transpose_w2(const lfric_op *op, const void *x, void *y);
