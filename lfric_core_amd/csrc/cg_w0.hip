@@ -31,7 +31,7 @@ __device__ inline Test test_of(const SolverState *st, const double *__restrict__
 // (record sets `done` while blocks of the apply start; a block it divides writes p and q alone, which a solve that
 // has ended does not read.)
 __device__ inline bool ended(SolverState *st, bool lead) {
-  if (!st->done && !st->status) return false;
+  if ((st->done | st->status) == 0) return false;  // one load of both
   if (lead) st->done = 1;
   return true;
 }
