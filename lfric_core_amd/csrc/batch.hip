@@ -614,7 +614,8 @@ constexpr double kEps = 2.220446049250313e-16;
 
 // Device buffers of destroyed batches and removed problems, kept for the next: a program that solves one batch
 // after another spent 4 of 23 ms (8 problems) in hipMalloc and hipFree.  Buffers come in size classes, eight
-// to a factor of two (at most 1/8 more than asked for), so that batches of similar sizes share them.  At most
+// to a factor of two (at most 1/8 more than asked for; exact beyond 1 GiB, which is never kept), so that
+// batches of similar sizes share them.  At most
 // 1 GiB in all; beyond that the longest-kept go, so sizes that do not recur leave again.  Kept buffers are no
 // live handle's (lfric_device_bytes): lfric_batch_kept_bytes counts them and lfric_batch_release_kept frees
 // them, as does an allocation of the library that fails.  Only idle buffers are put: their owners wait for the
@@ -625,6 +626,7 @@ size_t g_buf_bytes = 0;
 constexpr size_t kBufMax = size_t{1} << 30;
 
 size_t buf_class(size_t bytes) {
+  if (bytes > kBufMax) return bytes;  // never kept
   size_t step = 64;
   while (step * 16 < bytes) step *= 2;
   return std::max<size_t>((bytes + step - 1) / step * step, 64);

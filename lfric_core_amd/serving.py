@@ -53,6 +53,17 @@ def padded_rhs(nrhs):
     raise ValueError(nrhs)
 
 
+def batch_buffer_bytes(nbytes):
+    """Device bytes a batch takes for a buffer of nbytes: its size class, eight to a factor of two, up
+    to 1 GiB (batches share the buffers they leave behind by class); exact beyond."""
+    if nbytes > 1 << 30:
+        return nbytes
+    step = 64
+    while step * 16 < nbytes:
+        step *= 2
+    return max(-(-nbytes // step) * step, 64)
+
+
 def footprint_bytes(n, nl, order, nrhs):
     """Device bytes a request holds while admitted: FP64 and FP32 operators (level-aligned
     layout with 64-slot colour padding), the FP32 operator's batch copy (row-gathered for
@@ -71,8 +82,8 @@ def footprint_bytes(n, nl, order, nrhs):
         copy = (undf + 64) * 2 * 4 * 8 * 4
     else:
         units = nc * nl
-        copy = (units + 64) * 380 * 4 + units * 27 * 4 * (1 + r) + undf * 16
-    vecs = undf * r * (8 + 8 + 4 * 4 + 8) + undf * 4 * 2
+        copy = (units + 64) * 380 * 4 + units * 27 * 4 + batch_buffer_bytes(units * 27 * 4 * r) + undf * 16
+    vecs = undf * r * (8 + 8) + batch_buffer_bytes(undf * r * 4 * 4) + batch_buffer_bytes(undf * r * 8) + undf * 4 * 2
     maps = nc * ndf * 4 * 4
     return ops + copy + vecs + maps
 

@@ -192,3 +192,26 @@ def test_kept_buffers_are_bounded_and_follow_changing_sizes(hip):
     before = kept_bytes()
     assert add(64, 59, 8, 1) <= before - 24 * 8 * (6 * 64 * 64 + 2) * 60
     assert release_kept() <= limit and kept_bytes() == 0
+
+
+@pytest.mark.parametrize("n,nl,nrhs", [(5, 3, 1), (12, 20, 4), (24, 31, 2), (128, 86, 8)])
+def test_batch_buffers_take_their_class(hip, n, nl, nrhs):
+    """A problem's buffers take the bytes that the server's footprint counts: their size class, and exactly
+    what was asked for beyond 1 GiB (four FP32 vectors of C128x86 with 8 right-hand sides)."""
+    from lfric_core_amd.batch import Batch, release_kept
+    from lfric_core_amd.serving import batch_buffer_bytes
+    fs = hip.FunctionSpace.cubedsphere(n, nl)
+    op64, op32 = hip.LmaOperator(fs), hip.LmaOperator(fs, precision=hip.R32)
+    d32, x, b = hip.FieldVector(fs, hip.R32), hip.FieldVector(fs, hip.R64, nrhs), hip.FieldVector(fs, hip.R64, nrhs)
+    release_kept()
+    bt = Batch()
+    bt.add(op64, op32, d32, x, b)  # builds the space's lists
+    before = hip.device_bytes()
+    bt.add(op64, op32, d32, x, b)
+    vectors, residual = 16 * fs.undf * nrhs, 8 * fs.undf * nrhs
+    taken = batch_buffer_bytes(vectors) + batch_buffer_bytes(residual)
+    assert hip.device_bytes() - before == taken
+    assert vectors + residual <= taken <= 9 * (vectors + residual) / 8 + 64
+    assert vectors < 1 << 30 or batch_buffer_bytes(vectors) == vectors
+    bt.close()
+    release_kept()
