@@ -1,7 +1,6 @@
 // Conjugate gradient iteration over the element layout of a small lowest-order W0 operator, in two kernels.
 #include <hip/hip_runtime.h>
 
-#include "block_reduce.h"
 #include "device_common.h"
 #include "internal.h"
 #include "kernels.h"
@@ -10,6 +9,28 @@
 namespace lfric {
 namespace {
 
+// the sum of nb partials of NV values, in one fixed order in every block (for at most 8 kBlock of them the order of the
+// separate kernels' reduce_partials); 8 of a thread's are requested before any is added
+template <int NV>
+__device__ inline void sum_partials(const double *__restrict__ p, int nb, double (&tot)[NV]) {
+  constexpr int kU = 8;
+  double s[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) s[q] = 0.0;
+  for (int b = threadIdx.x; b < nb; b += kU * kBlock) {
+    double t[kU][NV];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int q = 0; q < NV; ++q) t[u][q] = b + u * kBlock < nb ? p[static_cast<size_t>(b + u * kBlock) * NV + q] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int q = 0; q < NV; ++q) s[q] += t[u][q];
+  }
+  block_sum<NV>(s, tot);
+}
+
 // ||r|| and r.z after the iterations so far (np partials of the update), and whether the solve ends with them
 struct Test {
   double rn, rz;
@@ -17,7 +38,7 @@ struct Test {
 };
 __device__ inline Test test_of(const SolverState *st, const double *__restrict__ partials, int np) {
   double tot[2];
-  sum_partials<kBlock, 2>(partials, np, tot);
+  sum_partials<2>(partials, np, tot);
   Test t;
   t.rn = sqrt(tot[0]);
   t.rz = tot[1];
@@ -152,7 +173,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_apply(const T *__restrict__ A,
     v[0] = to_d(acc) * to_d(p);
   }
   double tot[1];
-  block_sum_nt<kBlock, 1>(v, tot);
+  block_sum<1>(v, tot);
   if (threadIdx.x == 0) pq[blockIdx.x] = tot[0];
 }
 
@@ -169,7 +190,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_update(T *__restrict__ x, T *_
   const T xv = ok ? x[i] : T(0), rv = ok ? r[i] : T(0), pv = ok ? p[i] : T(0), qv = ok ? q[i] : T(0);
   const T dv = ok && diag ? diag[i] : T(1);
   double tp[1];
-  sum_partials<kBlock, 1>(pq, npq, tp);
+  sum_partials<1>(pq, npq, tp);
   const double pz = tp[0], alpha = st->rzb[it & 1] / pz;  // alpha = <r,z> / <p,A.p>
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   if (lead) st->pz = pz;
@@ -189,7 +210,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_w0_update(T *__restrict__ x, T *_
     v[1] = to_d(ri) * to_d(zi);
   }
   double tot[2];
-  block_sum_nt<kBlock, 2>(v, tot);
+  block_sum<2>(v, tot);
   if (threadIdx.x < 2) partials[2 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? tot[0] : tot[1];
 }
 
